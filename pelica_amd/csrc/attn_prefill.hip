@@ -25,6 +25,7 @@
 // one kv head (its K/V stays in that XCD's L2) and the longest key ranges
 // start first.
 #include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 
 #include "attn_prefill.hpp"
@@ -99,19 +100,32 @@ __device__ __forceinline__ unsigned long long rtime() { return __builtin_amdgcn_
 // stays resident in LDS, so the chunk loop has no tile waits and no
 // barriers; otherwise tiles stream through two K and two V buffers.
 // F32: f32 queries (rounded to f16 as they are loaded) and f32 output.
-template <int HD, int RT, bool RING, bool ROUND, int NW, int NRES = 0, bool F32 = false>
+// KG > 1 (streaming only): the waves form KG groups over the same rows, each
+// group walking its own contiguous share of the keys through its own K and V
+// buffers, TK keys a tile (64, or 32 where LDS holds no more); the groups'
+// (m, l, O) states are merged through LDS after the last chunk.
+template <int HD, int RT, bool RING, bool ROUND, int NW, int NRES = 0, bool F32 = false, int KG = 1, int TK = 64>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefillOcc<HD, RT>, kPrefillOcc<HD, RT>))) void prefill_kernel(
     PrefillParams p, int n_tb, int TB) {
     constexpr int KS = HD / 16;                 // 16-dim k-steps of QK^T
     constexpr int DT = HD / 32;                 // 32-dim output tiles
-    constexpr int TILE = 64 * HD * 2;           // bytes of a 64-key K (or V) tile
+    constexpr int TILE = TK * HD * 2;           // bytes of a K (or V) tile
+    constexpr int CPT = TK / 32;                // chunks per tile
+    constexpr int NWG = NW / KG;                // waves per key group
+    constexpr bool SPREAD = !NRES && !RING;     // the chunk loop's loads go out between its MFMAs
     constexpr int PPR = HD / 8;                 // 16-byte pieces per key row
     // streaming: K0 K1 V0 V1; resident: K[NRES] V[NRES] and a zero tile
     constexpr int NBUF = NRES ? 2 * NRES + 1 : 4;
-    static_assert(!NRES || !ROUND, "resident tiles: whole-cache launches only");
+    static_assert(!NRES || (!ROUND && KG == 1 && TK == 64), "resident tiles: whole-cache launches, one key group");
+    // (a share's chunks past klast: zeros past a linear cache's rows, but a
+    // ring's rows there may never have been written)
+    static_assert(!RING || KG == 1, "key groups: linear caches");
     // after the tile loop the f16 output of each wave is staged here
     constexpr int OUT_WAVE = RT * 32 * HD * 2;  // bytes of one wave's output rows
-    constexpr int LDS_BYTES = (ROUND || NBUF * TILE >= NW * OUT_WAVE) ? NBUF * TILE : NW * OUT_WAVE;
+    // key groups: every wave's O, then its (m, l), for the merge
+    constexpr int ST_O = NW * DT * RT * 64 * 64, ST_ML = NW * RT * 64 * 8;
+    constexpr int STREAM = KG * NBUF * TILE, AFTER = KG > 1 ? ST_O + ST_ML : ROUND ? 0 : NW * OUT_WAVE;
+    constexpr int LDS_BYTES = STREAM >= AFTER ? STREAM : AFTER;
     __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES];
 
     // XCD-aware block order: dispatch goes round-robin over the 8 XCDs, so
@@ -123,7 +137,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     const int rest = bid / n_tb;
     const int kvh = rest % p.n_kv, s = rest / p.n_kv;
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h2 = lane >> 5, c32 = lane & 31;
+    const int tid = threadIdx.x, wave = KG > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, lane = tid & 63,
+              h2 = lane >> 5, c32 = lane & 31;
+    const int kg = KG > 1 ? wave / NWG : 0, wr = KG > 1 ? wave % NWG : wave;  // key group, wave within it
 #ifdef PELICA_PTRACE
     const unsigned long long rt_entry = rtime();
     unsigned long long rt_loop0 = 0, rt_loop1 = 0, rt_issued = 0, rt_landed = 0, rt_bar = 0;
@@ -143,7 +159,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     // keys this launch covers: the whole cache, or one round's rows
     const int kbeg = ROUND ? p.key_begin : 0, kend = ROUND ? min(p.key_end, len) : len;
     const uint32_t stride_b = (uint32_t)p.row_stride * 2;
-    const uint32_t nrec = (RING ? (uint32_t)p.ring_cap : (uint32_t)(kend - kbeg)) * stride_b;
+    const int klast = min(pos_last, kend - 1);  // the last key a row sees
+    // (key groups: rows past klast, in a share's tail, read as zeros too)
+    const uint32_t nrec = (RING ? (uint32_t)p.ring_cap : (uint32_t)max(0, (KG > 1 ? klast + 1 : kend) - kbeg)) * stride_b;
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(p.k + row0 * p.row_stride + (size_t)kvh * HD), (short)0, (int)nrec, kBufferFlags);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
@@ -152,39 +170,48 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     // 64 keys start at kb0 (32-aligned), and the last tile may hold only one
     // needed chunk (a 32-token block of a window-128 layer takes 5 chunks, not
     // the 6 of 64-aligned whole tiles)
-    const int kb0 = max(lo_first, kbeg) & ~31;
-    const int klast = min(pos_last, kend - 1);
-    const int n_chunks = klast >= kb0 ? (klast - kb0) / 32 + 1 : 0;  // 0: a round past these tokens
-    const int n_tiles = (n_chunks + 1) / 2;
+    const int kb_all = max(lo_first, kbeg) & ~31;
+    const int n_all = klast >= kb_all ? (klast - kb_all) / 32 + 1 : 0;  // 0: a round past these tokens
+    // key groups take equal shares of the chunks (the barriers below keep
+    // them in step); what a share holds past klast is masked
+    const int n_chunks = KG > 1 ? (n_all + KG - 1) / KG : n_all;
+    const int kb0 = KG > 1 ? kb_all + 32 * n_chunks * kg : kb_all;
+    const int n_tiles = (n_chunks + CPT - 1) / CPT;
     // Tiles go from HBM straight into LDS (buffer_load ... lds): wave
     // instruction i of wave w fills LDS slots 64 (NW i + w) + lane (16 bytes
     // each) of a tile; the lane loads the logical piece that the swizzled
     // layout puts in its slot.
-    constexpr int WI = PPR / NW;  // wave instructions per tile and wave
-    static_assert(PPR % NW == 0, "tile pieces must split evenly over the waves");
-    char* const kbuf = lds;                            // K tiles
-    char* const vbuf = lds + (NRES ? NRES : 2) * TILE;  // V tiles
+    constexpr int WI = TK * PPR / 64 / NWG;  // wave instructions per tile and wave
+    static_assert(TK * PPR / 64 % NWG == 0, "tile pieces must split evenly over the waves");
+    char* const kbuf = lds + kg * NBUF * TILE;          // K tiles
+    char* const vbuf = kbuf + (NRES ? NRES : 2) * TILE;  // V tiles
     // buffer of tile t: its own (resident) or t & 1 (streaming)
     auto tbuf = [](int t) { return NRES ? t : (t & 1); };
     // tracked: the prologue's loads; the chunk loop's are untracked (the
     // compiler would wait for them before the PV's transposing V reads of
     // the same chunk; the loop waits for them itself, at the next barrier)
     auto load_tile = [&](const __amdgpu_buffer_rsrc_t& rs, char* dst, int tile, bool is_v, bool tracked) {
-        const int kb = kb0 + 64 * tile;
+        const int kb = kb0 + TK * tile;
 #pragma unroll
         for (int i = 0; i < WI; ++i) {
-            const int slot = 64 * (NW * i + wave) + lane;
+            const int slot = 64 * (NWG * i + wr) + lane;
             const int key = slot / PPR, phys = slot % PPR;
             const int piece = is_v ? phys ^ ((key & 3) << 1) : phys ^ (key & 7);
             // (round rows before key_begin wrap to offsets past nrec: zeros)
             const uint32_t off = RING ? ((kb + key) % p.ring_cap) * stride_b + 16 * piece
                                       : (uint32_t)(kb + key - kbeg) * stride_b + 16 * piece;
-            if (tracked) lds_dma16(rs, off, dst + 1024 * (NW * i + wave));
-            else lds_dma16_untracked(rs, off, dst + 1024 * (NW * i + wave));
+            if (tracked) lds_dma16(rs, off, dst + 1024 * (NWG * i + wr));
+            else lds_dma16_untracked(rs, off, dst + 1024 * (NWG * i + wr));
         }
     };
     // s_waitcnt vmcnt(0): the tile loads above have landed in LDS
     auto wait_tiles = [] { __builtin_amdgcn_s_waitcnt(0x0F70); };
+    // this wave's LDS reads are done, and no access moves across
+    auto wave_lds_done = [] {
+        __asm__ volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        __asm__ volatile("" ::: "memory");
+    };
 
     // The first tiles are requested before anything else, and nothing in
     // the prologue after them waits for a load: the queries come through a
@@ -198,8 +225,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     char* const vzero = NRES ? lds + 2 * NRES * TILE : vbuf + TILE;
     if (n_tiles > 0) {  // (uniform over the workgroup)
 #pragma unroll
-        for (int i = 0; i < TILE / (16 * 64 * NW); ++i)
-            *reinterpret_cast<u32x4*>(vzero + 16 * (tid + 64 * NW * i)) = u32x4{0, 0, 0, 0};
+        for (int i = 0; i < TILE / (16 * 64 * NWG); ++i)
+            *reinterpret_cast<u32x4*>(vzero + 16 * (64 * wr + lane + 64 * NWG * i)) = u32x4{0, 0, 0, 0};
         if (NRES) {
             // (the launch guarantees n_tiles <= NRES)
             for (int t = 0; t < n_tiles; ++t) load_tile(rk, kbuf + t * TILE, t, false, true);
@@ -207,7 +234,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         } else {
             load_tile(rk, kbuf, 0, false, true);
             if (n_tiles > 1) load_tile(rk, kbuf + TILE, 1, false, true);
-            load_tile(rv, vbuf, 0, true, true);
+            if (CPT == 2) load_tile(rv, vbuf, 0, true, true);
         }
     }
 
@@ -223,7 +250,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         (int)((uint32_t)(t1 - t0) * qtok_b), kBufferFlags);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-        const int r = (wave * RT + rt) * 32 + c32;
+        const int r = (wr * RT + rt) * 32 + c32;
         const int t = t0 + r / p.hpk;
         valid[rt] = r < TB * p.hpk && t < t1;
         const int h = kvh * p.hpk + r % p.hpk;
@@ -251,16 +278,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         m[rt] = valid[rt] ? -INFINITY : 0.f;  // rows past the block: all masked, fast path
         l[rt] = 0.f;
         if (!ROUND && p.sinks) {  // (every row's index is a head of this kv head)
-            const int r = (wave * RT + rt) * 32 + c32;
+            const int r = (wr * RT + rt) * 32 + c32;
             const float sk = p.sinks[kvh * p.hpk + r % p.hpk] * kLog2e;
-            m[rt] = valid[rt] ? sk : m[rt];
-            l[rt] = valid[rt] && h2 == 0 ? 1.f : 0.f;
+            m[rt] = valid[rt] && kg == 0 ? sk : m[rt];
+            l[rt] = valid[rt] && kg == 0 && h2 == 0 ? 1.f : 0.f;
         }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[dt][rt] = float16v{};
-        if (ROUND && !p.first && valid[rt]) {
+        if (ROUND && !p.first && valid[rt] && kg == 0) {
             // the running state of the rounds before (sum split over h2 lanes)
-            const int r = (wave * RT + rt) * 32 + c32;
+            const int r = (wr * RT + rt) * 32 + c32;
             const int t = t0 + r / p.hpk, h = kvh * p.hpk + r % p.hpk;
             const float* st = p.state + ((size_t)(s * p.T + t) * p.n_head + h) * (HD + 2);
             m[rt] = st[0] <= -1.0e38f ? -INFINITY : st[0] * kLog2e;
@@ -275,8 +302,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     // S^T of chunk c (32 keys x RT row tiles): element i of a lane is key
     // 32 c + 8 (i / 4) + 4 h2 + i % 4 of row c32
     auto qk = [&](int c, float16v (&sc)[RT]) {
-        const char* kt = kbuf + tbuf(c >> 1) * TILE;
-        const int krow = 32 * (c & 1) + c32;
+        const char* kt = kbuf + tbuf(c / CPT) * TILE;
+        const int krow = 32 * (c % CPT) + c32;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) sc[rt] = float16v{};
 #pragma unroll
@@ -288,7 +315,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     };
     // O^T += V^T P^T over chunk c; pb[w] holds keys 16 w .. 16 w + 15 of it
     auto pv = [&](int c, const half8 (&pb)[2][RT]) {
-        const char* vt = vbuf + tbuf(c >> 1) * TILE;
+        const char* vt = vbuf + tbuf(c / CPT) * TILE;
         const int G = lane >> 4, r4 = (lane & 15) >> 2, q4 = lane & 3;
 #pragma unroll
         for (int w = 0; w < 2; ++w) {
@@ -297,7 +324,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
             for (int dt = 0; dt < DT; ++dt) {
                 // lanes of 16-lane group G read keys 16w + 4 h2 + r (+8) at
                 // dims 32 dt + 16 (G & 1) + 4 q; lane 4r + q of the group
-                const int key = 32 * (c & 1) + 16 * w + 4 * h2 + r4, dim = 32 * dt + 16 * (G & 1) + 4 * q4;
+                const int key = 32 * (c % CPT) + 16 * w + 4 * h2 + r4, dim = 32 * dt + 16 * (G & 1) + 4 * q4;
                 const _Float16* a0 = reinterpret_cast<const _Float16*>(vt + v_slot<HD>(key, dim >> 3) + ((dim & 7) << 1));
                 const _Float16* a1 = reinterpret_cast<const _Float16*>(vt + v_slot<HD>(key + 8, dim >> 3) + ((dim & 7) << 1));
                 va[dt] = cat8(lds_read_tr(a0), lds_read_tr(a1));
@@ -348,6 +375,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) p_b[w][rt] = half8{0, 0, 0, 0, 0, 0, 0, 0};
     qk(0, s_a);
+    if (CPT == 1) {  // chunk 0's step refills K tile 0's buffer
+        if (NWG > 1) __syncthreads();
+        else wave_lds_done();
+    }
     const half2 one2 = {(_Float16)1.f, (_Float16)1.f};
 
     // one chunk: scores of c in s_cur, of c+1 into s_nxt; P of c-1 in
@@ -360,11 +391,31 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         constexpr int PAR = decltype(par)::value;
         // K of tile t+2 and V of tile t+1 at odd chunks c = 2t+1: their
         // buffers' last readers finished at chunk 2t; first readers at 2t+3
-        const int t = c >> 1;
-        if (!NRES && (PAR & 1)) {
+        // (32-key tiles: K of chunk c+2 and V of chunk c, whose buffers'
+        // last readers finished at chunk c-1; first readers at c+1)
+        const int t = c / CPT;
+        if (!NRES && !SPREAD && (PAR & 1)) {
             if (t + 2 < n_tiles) load_tile(rk, kbuf + (t & 1) * TILE, t + 2, false, false);
             if (t + 1 < n_tiles) load_tile(rv, vbuf + ((t + 1) & 1) * TILE, t + 1, true, false);
         }
+        // SPREAD: one load at a time beside the MFMAs of the first LSL
+        // slots (below), not a burst here: a wave stalls at each until the
+        // memory pipeline takes it, with its first MFMAs behind it (clocks
+        // per 32-key chunk, one group / four groups: head dim 64 1966 / 2490
+        // -> 1900 / 2064, head dim 128 1826 / 2400 -> 1722 / 2100).  No
+        // branches there either (they cost more than the burst): a tile past
+        // the last one is requested past the rows, which reads nothing.
+        constexpr int NLD = SPREAD && (CPT == 1 || (PAR & 1)) ? 2 * WI : 0;
+        const int tk = t + 2, tv = t + CPT - 1;
+        const uint32_t off_k = tk < n_tiles ? (uint32_t)(kb0 + TK * tk - kbeg) * stride_b : 0xF0000000u;
+        const uint32_t off_v = tv < n_tiles ? (uint32_t)(kb0 + TK * tv - kbeg) * stride_b : 0xF0000000u;
+        auto load_nth = [&](int n) {
+            const bool is_v = n >= WI;
+            const int i = is_v ? n - WI : n, slot = 64 * (NWG * i + wr) + lane, key = slot / PPR, phys = slot % PPR;
+            const int piece = is_v ? phys ^ ((key & 3) << 1) : phys ^ (key & 7);
+            lds_dma16_untracked(is_v ? rv : rk, (is_v ? off_v : off_k) + (uint32_t)key * stride_b + 16 * piece,
+                                (is_v ? vbuf + (tv & 1) * TILE : kbuf + (tk & 1) * TILE) + 1024 * (NWG * i + wr));
+        };
 
         const int kb = kb0 + 32 * c;
         if (kb + 31 > pos_first || kb < lo_last || (ROUND && (kb < kbeg || kb + 31 >= kend))) {
@@ -384,11 +435,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         constexpr int NOPD = KS + 2 * DT;
         half8 opd[NOPD];
         // (resident tiles: PAR = c itself)
-        const char* const kt_c = kbuf + (NRES ? ((PAR + 1) >> 1) : (((PAR + 1) >> 1) & 1)) * TILE;
-        const int krow = 32 * ((PAR + 1) & 1) + c32;
+        const char* const kt_c = kbuf + (NRES ? ((PAR + 1) >> 1) : (((PAR + 1) / CPT) & 1)) * TILE;
+        const int krow = 32 * ((PAR + 1) % CPT) + c32;
         // chunk c-1 (c = 0: the zeroed tile)
         const char* const vt_c = NRES ? (PAR == 0 ? vzero : vbuf + ((PAR - 1) >> 1) * TILE)
-                                      : vbuf + (((PAR + 3) >> 1) & 1) * TILE;
+                                      : vbuf + (((PAR + 3) / CPT) & 1) * TILE;
         auto read_opd = [&](int r) {
             if (r < KS) {
                 opd[r] = *reinterpret_cast<const half8*>(kt_c + k_slot<HD>(krow, 2 * r + h2));
@@ -397,7 +448,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
                 // dims 32 dt + 16 (G & 1) + 4 q4; lane 4 r4 + q4 of the group
                 const int w = (r - KS) / DT, dt = (r - KS) % DT;
                 const int G = lane >> 4, r4 = (lane & 15) >> 2, q4 = lane & 3;
-                const int key = 32 * ((PAR + 3) & 1) + 16 * w + 4 * h2 + r4, dim = 32 * dt + 16 * (G & 1) + 4 * q4;
+                const int key = 32 * ((PAR + 3) % CPT) + 16 * w + 4 * h2 + r4, dim = 32 * dt + 16 * (G & 1) + 4 * q4;
                 const _Float16* a0 = reinterpret_cast<const _Float16*>(vt_c + v_slot<HD>(key, dim >> 3) + ((dim & 7) << 1));
                 const _Float16* a1 = reinterpret_cast<const _Float16*>(vt_c + v_slot<HD>(key + 8, dim >> 3) + ((dim & 7) << 1));
                 opd[r] = cat8(lds_read_tr(a0), lds_read_tr(a1));
@@ -417,6 +468,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         // dots of the pairs packed in slot t-1, so every 32-cycle MFMA has
         // the same small mix of vector work beside it (S scores per slot).
         constexpr int NM = KS * RT + 2 * DT * RT;  // MFMAs
+        // slots the loads go out in: half of them, or all where that still
+        // leaves them a whole chunk to land
+        constexpr int LSL = HD == 128 && CPT == 2 ? NM : NM / 2;
         constexpr int NS = 16 * RT;                // scores per lane
         constexpr int NP = NS / 2;                 // score pairs
         static_assert(NS % NM == 0, "whole scores per MFMA slot");
@@ -454,6 +508,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         for (int t = 0; t < NM; ++t) {
             const int r = t / RT;  // operand of MFMA t
             if (t % RT == 0 && r + 2 < NOPD) read_opd(r + 2);
+            if (SPREAD) {
+#pragma unroll
+                for (int i = t * NLD / LSL; i < (t + 1) * NLD / LSL && i < NLD; ++i) load_nth(i);
+            }
             // 8-wave workgroups: the wave about to issue its MFMA takes
             // issue priority over its SIMD partner's vector work (the
             // 4096-token gpt-oss causal prefill ~1.7 % faster; 4-wave
@@ -522,7 +580,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         // chunk 2t, and (b) the loads of chunk 2t-1 are first read at chunk
         // 2t+1, so they must have landed (vmcnt(0)) before it.  Chunk 2t+1
         // reads only tiles published by this barrier or earlier ones.
-        if (!NRES && (PAR & 1) == 0) {
+        // (32-key tiles: a barrier after every chunk.)
+        if (!NRES && (CPT == 1 || (PAR & 1) == 0)) {
 #ifdef PELICA_PTRACE
             const unsigned ta = cyc();
             wait_tiles();
@@ -532,7 +591,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
             t_bar += cyc() - tb2;
 #else
             wait_tiles();
-            __syncthreads();
+            if (NWG > 1) __syncthreads();
+            else wave_lds_done();  // (a group of one wave: its own buffers, no one to wait for)
 #endif
         }
 #ifdef PELICA_PTRACE
@@ -579,6 +639,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     if (rem >= 1) step(P0{}, c, s_a, s_b, p_b, p_a);
     if (rem >= 2) step(P1{}, c + 1, s_b, s_a, p_a, p_b);
     if (rem >= 3) step(P2{}, c + 2, s_a, s_b, p_b, p_a);
+    if (SPREAD) wait_tiles();  // (requests past the last tile write zeros to a buffer no one reads)
     if (rem & 1) pv(n_chunks - 1, p_a);
     else pv(n_chunks - 1, p_b);
     }
@@ -594,7 +655,85 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
 #endif
     }
 
-    if constexpr (!ROUND && F32) {
+    if constexpr (KG > 1) {
+        // The groups' states, merged in key order.  Every wave leaves its
+        // O and (m, l) in LDS; group g then takes the output tiles
+        // j = g * TPG ... of its rows, summed over the groups (each lane
+        // reads what its counterparts wrote: 16-byte accesses, no conflicts).
+        constexpr int TPG = DT * RT / KG > 0 ? DT * RT / KG : 1;  // tiles per group
+        float4v* const so = reinterpret_cast<float4v*>(lds);
+        float2* const sml = reinterpret_cast<float2*>(lds + ST_O);
+        __syncthreads();  // every wave is done with the K/V tiles
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            sml[(wave * RT + rt) * 64 + lane] = make_float2(m[rt], half_sum(l[rt]));
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4)
+                    so[((wave * DT * RT + dt * RT + rt) * 4 + i4) * 64 + lane] =
+                        float4v{o[dt][rt][4 * i4], o[dt][rt][4 * i4 + 1], o[dt][rt][4 * i4 + 2], o[dt][rt][4 * i4 + 3]};
+        }
+        __syncthreads();
+        if (kg * TPG >= DT * RT) return;
+#pragma unroll
+        for (int jj = 0; jj < TPG; ++jj) {
+            const int j = kg * TPG + jj, dt = j / RT, rt = j % RT;
+            const int r = (wr * RT + rt) * 32 + c32;
+            const int t = t0 + r / p.hpk, h = kvh * p.hpk + r % p.hpk;
+            if (r >= TB * p.hpk || t >= t1) continue;
+            float2 ml[KG];
+            float M = -INFINITY;
+#pragma unroll
+            for (int g = 0; g < KG; ++g) {
+                ml[g] = sml[((g * NWG + wr) * RT + rt) * 64 + lane];
+                M = fmaxf(M, ml[g].x);
+            }
+            const float ms = M == -INFINITY ? 0.f : M;
+            float L = 0.f;
+            float4v ov[4] = {};
+#pragma unroll
+            for (int g = 0; g < KG; ++g) {
+                const float w = fast_exp2(ml[g].x - ms);  // 0 where the group saw no key
+                L += ml[g].y * w;
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) ov[i4] += so[(((g * NWG + wr) * DT * RT + j) * 4 + i4) * 64 + lane] * w;
+            }
+            float inv = 1.f / L;
+            if constexpr (ROUND) {
+                float* st = p.state + ((size_t)(s * p.T + t) * p.n_head + h) * (HD + 2);
+                if (h2 == 0 && dt == 0) {
+                    st[0] = M == -INFINITY ? -3.0e38f : M * kLn2;
+                    st[1] = L;
+                }
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) st[2 + 32 * dt + 8 * i4 + 4 * h2 + i] = ov[i4][i];
+                if (!p.out) continue;
+                // the output so far: sink in max and denominator; 0 before any key
+                if (p.sinks) {
+                    const float sk = p.sinks[h] * kLog2e;
+                    const float M2 = fmaxf(M, sk);
+                    const float w = M == -INFINITY ? 0.f : fast_exp2(M - M2);
+                    inv = w / (L * w + fast_exp2(sk - M2));
+                } else {
+                    inv = L > 0.f ? inv : 0.f;
+                }
+            }
+            const size_t ob = (size_t)(s * p.T + t) * p.o_tok + h * HD + 32 * dt + 4 * h2;
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) {
+                const float4v x = ov[i4] * inv;
+                if constexpr (F32) {
+                    *reinterpret_cast<float4v*>(static_cast<float*>(p.out) + ob + 8 * i4) = x;
+                } else {
+                    const half4 hv = {(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
+                    *reinterpret_cast<half4*>(static_cast<uint16_t*>(p.out) + ob + 8 * i4) = hv;
+                }
+            }
+        }
+    } else if constexpr (!ROUND && F32) {
         // f32 output: each lane stores its rows' 16-byte pieces
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
@@ -1186,11 +1325,80 @@ static int window_tiles(int window, int TB) {
     return (chunks + 1) / 2;
 }
 
+static int prefill_cus() {
+    static const int n = [] {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+            cus = 256;
+        return cus;
+    }();
+    return n;
+}
+
+// How an 8-wave launch cuts its work: `split` 1 is one key group per
+// workgroup on all of its rows; each step halves a workgroup's rows and
+// doubles the number of workgroups: key groups 2, 4 and (head dim 64) 8, then
+// (16) eight groups with one row tile a wave.  Few rows leave most CUs idle
+// otherwise: 512 gpt-oss tokens are 64 workgroups of 512 rows, and a full
+// layer at position 30K took 772 us with 1 group, 414 with 2, 278 with 4, 317
+// with 8 (512 workgroups: two generations); 256 Qwen3 tokens over 27K keys
+// (two rounds) 635 / 331 / 224; 64 gpt-oss tokens at 8K 204 / 110 / 62 / 40 /
+// 27.5.  Where the grid fills the chip anyway, groups only cost: each loads
+// its own keys (LDS writes beside the operand reads), and every workgroup
+// pays its start and its merge (4096 fresh gpt-oss tokens 147 / 164 / 205 /
+// 281 us).  So the split with the least estimated time is taken, from what
+// these shapes measured: us per key a group walks and us per workgroup, with
+// most CUs idle (lat) and with all of them busy (thr: lower clock, shared
+// memory rates).
+struct SplitCost {
+    float key_lat, wg_lat, key_thr, wg_thr;
+};
+constexpr SplitCost kSplitCost64[5] = {{.0244f, 3.5f, .0325f, 4.0f}, {.0246f, 5.5f, .0330f, 6.8f}, {.0285f, 6.0f, .0350f, 8.0f},
+                                       {.0300f, 6.0f, .0370f, 8.0f}, {.0250f, 3.0f, .0250f, 4.8f}};
+constexpr SplitCost kSplitCost128[3] = {{.0232f, 4.0f, .0375f, 4.0f}, {.0240f, 5.0f, .0385f, 7.0f}, {.0325f, 5.0f, .0407f, 8.0f}};
+
+static int prefill_split(const PrefillParams& p, int rows) {
+#ifdef KG_ENV
+    if (const char* e = getenv("PELICA_KG")) return atoi(e);
+#endif
+    const SplitCost* const cost = p.hd == 64 ? kSplitCost64 : kSplitCost128;
+    const int n_split = p.hd == 64 ? 5 : 3;
+    const double cus = prefill_cus();
+    // keys of the longest token block, and how many fewer the shortest walks
+    const double keys = p.state ? p.key_end - p.key_begin : p.kv_len;
+    const double spread = std::min<double>(p.state ? std::max(0, p.T - (p.kv_len - p.key_end)) : p.T, keys);
+    const long long same = (long long)p.n_kv * p.n_seq;  // blocks of one length
+    // (the last share's masked tail stays inside 32-bit offsets)
+    const bool fits = ((long long)p.kv_len + 512) * p.row_stride * 2 < 1LL << 32;
+    double best = 0;
+    int pick = 1;
+    for (int i = 0; i < n_split; ++i) {
+        const int split = 1 << i, TB = rows / split / p.hpk, kg = std::min(split, 8);
+        if (TB == 0 || (i > 0 && !fits)) break;
+        const long long n_tb = (p.T + TB - 1) / TB, n = n_tb * same;
+        auto walk = [&](long long b) { return (keys - (double)(b / same) / n_tb * spread) / kg; };  // block b, longest first
+        const SplitCost& c = cost[i];
+        // the longest block (at the clock of a chip whose CUs are busy that
+        // share of the time) ...
+        const double mean = (keys - spread / 2) / kg, busy = std::min(1.0, n / cus * mean / walk(0));
+        const double per_key = c.key_lat + (c.key_thr - c.key_lat) * std::max(0.0, 2 * busy - 1);
+        double t = walk(0) * per_key + c.wg_lat;
+        // ... all the work over all CUs ...
+        if (n >= cus) t = std::max(t, n / cus * (mean * c.key_thr + c.wg_thr));
+        // ... and g + 1 of the first g * cus + 1 blocks on one CU
+        for (int g = 1; g <= 8 && g * cus < n; ++g) t = std::max(t, (g + 1) * (walk((long long)(g * cus)) * c.key_lat + c.wg_lat));
+        if (i == 0 || 1.05 * t < best) best = t, pick = split;
+    }
+    return pick;
+}
+
 template <int HD, int RT, int NW, bool F32>
 static hipError_t launch_nw(const PrefillParams& p, hipStream_t st) {
     constexpr int ROWS = NW * RT * 32;
     if (p.hpk > ROWS) return hipErrorNotSupported;
-    const int TB = ROWS / p.hpk;
+    const int split = NW == 8 && !p.ring_cap ? prefill_split(p, ROWS) : 1, KG = std::min(split, 8);
+    const int TB = ROWS / split / p.hpk;
     const int n_tb = (p.T + TB - 1) / TB;
     const long long nblk = (long long)n_tb * p.n_kv * p.n_seq;
     if (nblk > 0x7fffffff) return hipErrorNotSupported;
@@ -1204,6 +1412,25 @@ static hipError_t launch_nw(const PrefillParams& p, hipStream_t st) {
         if (res) {
             if (p.ring_cap) hipLaunchKernelGGL((prefill_kernel<HD, RT, true, false, NW, 3, F32>), grid, block, 0, st, p, n_tb, TB);
             else hipLaunchKernelGGL((prefill_kernel<HD, RT, false, false, NW, 3, F32>), grid, block, 0, st, p, n_tb, TB);
+            return hipGetLastError();
+        }
+    }
+    if constexpr (NW == 8) {
+        constexpr int TK4 = HD == 64 ? 64 : 32;  // (4 groups of 64-key tiles of 128 dims: past the LDS)
+        if (KG > 1) {
+            auto go = [&](auto rt, auto kg, auto tk) {
+                constexpr int R = decltype(rt)::value, G = decltype(kg)::value, K = decltype(tk)::value;
+                if (p.state) hipLaunchKernelGGL((prefill_kernel<HD, R, false, true, NW, 0, F32, G, K>), grid, block, 0, st, p, n_tb, TB);
+                else hipLaunchKernelGGL((prefill_kernel<HD, R, false, false, NW, 0, F32, G, K>), grid, block, 0, st, p, n_tb, TB);
+            };
+            using std::integral_constant;
+            using RTc = integral_constant<int, RT>;
+            if (KG == 2) go(RTc{}, integral_constant<int, 2>{}, integral_constant<int, 64>{});
+            else if (KG == 4) go(RTc{}, integral_constant<int, 4>{}, integral_constant<int, TK4>{});
+            else if constexpr (HD == 64) {
+                if (split == 8) go(RTc{}, integral_constant<int, 8>{}, integral_constant<int, 32>{});
+                else go(integral_constant<int, 1>{}, integral_constant<int, 8>{}, integral_constant<int, 32>{});
+            }
             return hipGetLastError();
         }
     }
@@ -1223,17 +1450,6 @@ static hipError_t launch_nw(const PrefillParams& p, hipStream_t st) {
 // ring slots of the sliding-window kernel: the chunks of two consecutive
 // 64-token blocks, (126 + window) / 32 + 2, fit for windows up to 130
 constexpr int kSlideChunks = 10;
-
-static int prefill_cus() {
-    static const int n = [] {
-        int dev = 0, cus = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
-        return cus;
-    }();
-    return n;
-}
 
 // the sliding-window kernel's shapes: head dim 64, 8 heads per kv head,
 // whole-prompt launches, a window its chunk ring holds

@@ -184,3 +184,46 @@ def test_slide_window_ring_ragged_sequences():
                         seq_kv_offset=np.array([0, cap], dtype=np.int64), sinks=inp.sinks.cpu().numpy(), window=W,
                         ring_cap=cap)
     assert_close(as_f64(got), as_f64(ref), what="slide ring ragged")
+
+
+@pytest.mark.parametrize("hd,n_head,n_kv,T,L,n_seq,ragged,window", [
+    (64, 64, 8, 20, 1500, 1, None, 0),      # eight key groups on one row tile (32 rows)
+    (64, 24, 8, 33, 700, 1, None, 0),       # ... of 30 rows in 32 (3 heads per kv head)
+    (64, 40, 1, 9, 600, 1, None, 0),        # more heads per kv head than a 32-row workgroup holds
+    (64, 64, 8, 250, 5250, 1, None, 0),     # eight groups
+    (64, 64, 8, 300, 311, 1, None, 0),      # four
+    (64, 64, 8, 700, 700, 2, None, 0),      # two
+    (64, 64, 8, 5, 5, 1, None, 0),          # one chunk: every group but the first walks nothing
+    (64, 64, 8, 100, 3000, 1, None, 1500),  # a window too long for the short-window kernels
+    (128, 32, 4, 256, 256, 1, None, 0),     # head dim 128: four groups of 32-key tiles
+    (128, 16, 16, 33, 2049, 1, None, 0),    # ... an odd share of the chunks
+    (128, 32, 4, 1000, 1000, 1, None, 0),   # two groups
+    (128, 32, 4, 40, 3000, 3, (40, 3000), 0),   # ragged: short sequences leave whole groups without keys
+])
+@pytest.mark.parametrize("f32", [False, True])
+def test_key_groups(hd, n_head, n_kv, T, L, n_seq, ragged, window, f32):
+    cfg = wl.AttnConfig("pkg", "prefill", n_head, n_kv, hd, L, q_tokens=T, n_seq=n_seq, ragged=ragged, window=window,
+                        sinks=hd == 64, seed=hd + T + L)
+    inp = wl.make_inputs(cfg, "cuda")
+    print(f"[case] key groups hd{hd} h{n_head}/{n_kv} T{T} L{L} n_seq{n_seq} window{window} f32 {f32}", flush=True)
+    ref = as_f64(oracle_run(inp))
+    if f32:
+        inp.q = inp.q.float()
+    assert_close(as_f64(gpu_run(inp)), ref, what="key groups")
+
+
+@pytest.mark.parametrize("hd,n_head,n_kv,T,L,bounds,window", [
+    (64, 64, 8, 40, 3000, [0, 1, 700, 2980, 3000], 0),   # a last round that only some tokens see
+    (64, 64, 8, 250, 6000, [0, 5000, 5800, 6000], 0),
+    (128, 32, 4, 100, 5000, [0, 777, 3000, 5000], 0),
+    (64, 64, 8, 64, 4000, [0, 1500, 4000], 1600),
+])
+def test_key_groups_in_rounds(hd, n_head, n_kv, T, L, bounds, window):
+    from tests.test_gpu_prefill_rounds import run_rounds
+
+    cfg = wl.AttnConfig("pkr", "prefill", n_head, n_kv, hd, L, q_tokens=T, window=window, sinks=True, seed=T + L)
+    inp = wl.make_inputs(cfg, "cuda")
+    print(f"[case] key groups in rounds hd{hd} T{T} L{L} {bounds} window{window}", flush=True)
+    out, state = run_rounds(inp, bounds, window=window)
+    assert_close(as_f64(out), as_f64(oracle_run(inp)), what="key groups in rounds")
+    assert torch.isfinite(state).all()
