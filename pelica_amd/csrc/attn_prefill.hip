@@ -1477,6 +1477,20 @@ static hipError_t launch_slide(const PrefillParams& p, hipStream_t st) {
 
 template <int HD, int RT, bool F32>
 static hipError_t launch(const PrefillParams& p, hipStream_t st) {
+    if constexpr (HD == 64) {
+        // Short windows, few tokens: one row tile a wave, half the rows a
+        // workgroup.  Every wave's chunks then take half as long, which is
+        // what such a call waits for, and the grid reaches twice the CUs
+        // (gpt-oss window 128, f32 / f16: 512 tokens 13.9 / 12.3 -> 9.4 / 6.8
+        // us, 1024 14.8 / 13.0 -> 12.5 / 9.2, 1600 18.7 / 14.2 -> 18.1 / 13.8;
+        // past three workgroups a CU the two-tile kernels, whose rows share
+        // each K/V tile among more of them: 2048 tokens 20.4 / 14.4 against
+        // 21.3 / 16.0).
+        if (p.window > 0 && p.window <= 1024 && p.hpk <= 128) {
+            const int TB = 128 / p.hpk;
+            if ((long long)((p.T + TB - 1) / TB) * p.n_kv * p.n_seq <= 3LL * prefill_cus()) return launch_nw<HD, 1, 4, F32>(p, st);
+        }
+    }
     if (HD == 64 && RT == 2 && !F32 && slide_fits(p)) return launch_slide(p, st);
     if (p.window > 0 && p.window <= 1024) return launch_nw<HD, RT, 4, F32>(p, st);
     return launch_nw<HD, RT, 8, F32>(p, st);

@@ -227,3 +227,25 @@ def test_key_groups_in_rounds(hd, n_head, n_kv, T, L, bounds, window):
     out, state = run_rounds(inp, bounds, window=window)
     assert_close(as_f64(out), as_f64(oracle_run(inp)), what="key groups in rounds")
     assert torch.isfinite(state).all()
+
+
+@pytest.mark.parametrize("T,L,window,n_seq,n_head,f32", [
+    (1, 300, 128, 1, 64, False),      # one row tile a wave, one token
+    (17, 17, 128, 1, 64, True),       # 16-token blocks and one token more
+    (500, 2000, 100, 2, 64, False),
+    (300, 1500, 1000, 1, 64, True),   # a window whose tiles stream
+    (130, 400, 64, 1, 24, True),      # 3 heads per kv head: 126 rows of 128
+    (1536, 1536, 128, 1, 64, True),   # the most tokens of one row tile a wave
+    (1537, 1600, 128, 1, 64, True),   # one more: two row tiles
+    (1537, 1600, 128, 1, 64, False),  # ... and the sliding-window kernel, ragged last block
+    (700, 1100, 130, 3, 64, False),
+])
+def test_short_window_row_tiles(T, L, window, n_seq, n_head, f32):
+    cfg = wl.AttnConfig("pwr", "prefill", n_head, 8, 64, L, q_tokens=T, n_seq=n_seq, window=window, sinks=True,
+                        ragged=(T, L) if n_seq > 1 else None, seed=T + L)
+    inp = wl.make_inputs(cfg, "cuda")
+    print(f"[case] short window T{T} L{L} window{window} n_seq{n_seq} h{n_head} f32 {f32}", flush=True)
+    ref = as_f64(oracle_run(inp))
+    if f32:
+        inp.q = inp.q.float()
+    assert_close(as_f64(gpu_run(inp)), ref, what="short window")
