@@ -9,6 +9,8 @@
 // 64/(hd/4) slots of a few consecutive tokens.  The norm is a reduction over the slot's lanes; the
 // rotation reads each element's partner through the slot's LDS row.
 // HBM-bound: every byte is touched once.
+#include <type_traits>
+
 #include "attn_prof.hpp"
 #include "attn_qkv.hpp"
 
@@ -160,7 +162,108 @@ __global__ __launch_bounds__(256) void qkv_rope_cache_kernel(QkvParams p) {
     }
 }
 
-// tokens per wave (gpt-oss 4096-token step: 1 token 34.7 us, 2 30.3, 3 30.3,
+// The same step where every access can be 16 bytes wide (QkvParams::wide): a
+// wave takes one token and IT groups of 64/(HD/4) consecutive heads; the
+// token's rotation is loaded in 16-byte pieces, once for all of its groups,
+// and a rotation partner comes from its lane's registers, not through LDS.
+// Small steps are one dependent chain of load, exchange and store: fewer
+// instructions and more waves shorten it; large ones run at the copy rate.
+template <int HD, int IT>
+__global__ __launch_bounds__(256) void qkv_rope_cache_wide_kernel(QkvParams p) {
+    constexpr int LPH = HD / 4, HPW = 64 / LPH;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane / LPH, e0 = 4 * (lane % LPH);
+    const int t = blockIdx.y, s = blockIdx.z, n_slot = p.n_head + 2 * p.n_kv;
+    const int slot0 = (blockIdx.x * 4 + wave) * (HPW * IT) + sub;
+    if (slot0 - sub >= n_slot) return;
+    const int len = seq_keys(p.seq_len, s, p.kv_len);
+    if (len < p.T || len > p.kv_len) return;  // (attention skips such sequences too)
+    const size_t tok = (size_t)s * p.T + t;
+    const int pos = len - p.T + t, half = p.rot / 2;
+    float4v x[IT];
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int slot = min(slot0 + HPW * it, n_slot - 1);  // (slots past the end store nothing)
+        const int hk = slot - p.n_head, hv = hk - p.n_kv;
+        const float* src = hk < 0 ? p.q + tok * p.tok_q + (size_t)slot * HD
+                                  : (hv < 0 ? p.k + (size_t)hk * HD : p.v + (size_t)hv * HD) + tok * p.tok_kv;
+        x[it] = *reinterpret_cast<const float4v*>(src + e0);
+    }
+    const float4v wq = p.q_norm ? *reinterpret_cast<const float4v*>(p.q_norm + e0) : float4v{1.f, 1.f, 1.f, 1.f};
+    const float4v wk = p.k_norm ? *reinterpret_cast<const float4v*>(p.k_norm + e0) : float4v{1.f, 1.f, 1.f, 1.f};
+    // cos, sin of this lane's elements: 4 pairs (NeoX) or 2 (interleaved)
+    const bool rot = e0 < p.rot;
+    const bool hi = p.neox && e0 >= half;  // the second element of its pairs
+    float c[4] = {1.f, 1.f, 1.f, 1.f}, sn[4] = {0.f, 0.f, 0.f, 0.f};
+    if (rot) {
+        const int j = p.neox ? (hi ? e0 - half : e0) : e0 >> 1;
+        auto row = [&](size_t r, float (&cc)[4], float (&ss)[4]) {
+            const float4v* q = reinterpret_cast<const float4v*>(p.table + (r * half + j) * 2);
+            const float4v a = q[0], b = p.neox ? q[1] : a;
+            if (p.neox) {
+                cc[0] = a[0], ss[0] = a[1], cc[1] = a[2], ss[1] = a[3];
+                cc[2] = b[0], ss[2] = b[1], cc[3] = b[2], ss[3] = b[3];
+            } else {
+                cc[0] = cc[1] = a[0], ss[0] = ss[1] = a[1], cc[2] = cc[3] = a[2], ss[2] = ss[3] = a[3];
+            }
+        };
+        if (p.table_split <= 0) {
+            row(pos, c, sn);
+        } else {
+            float c1[4], s1[4], c2[4], s2[4];
+            row(pos >> 8, c1, s1);
+            row(p.table_split + (pos & 255), c2, s2);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                c[i] = c1[i] * c2[i] - s1[i] * s2[i];
+                sn[i] = s1[i] * c2[i] + c1[i] * s2[i];
+            }
+        }
+    }
+    const int partner = !rot || !p.neox ? lane : hi ? lane - half / 4 : lane + half / 4;
+    const int64_t base = p.seq_off ? p.seq_off[s] : (int64_t)s * (p.ring_cap ? p.ring_cap : p.kv_len);
+    const int64_t rowi = base + (p.ring_cap ? pos % p.ring_cap : pos);
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int slot = slot0 + HPW * it, hk = slot - p.n_head, hv = hk - p.n_kv;
+        float4v y = x[it];
+        if (p.q_norm || p.k_norm) {
+            float ss = y[0] * y[0] + y[1] * y[1] + y[2] * y[2] + y[3] * y[3];
+#pragma unroll
+            for (int off = LPH / 2; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
+            if (hk < 0 ? p.q_norm != nullptr : hv < 0 && p.k_norm) {
+                const float inv = 1.f / __builtin_sqrtf(ss / (float)HD + p.eps);
+                const float4v w = hk < 0 ? wq : wk;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[i] = y[i] * inv * w[i];
+            }
+        }
+        if (p.table) {
+            float4v z;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) z[i] = p.neox ? __shfl(y[i], partner, 64) : y[i ^ 1];
+            if (rot && hv < 0) {
+                float4v r;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const bool second = p.neox ? hi : (i & 1) != 0;
+                    r[i] = second ? z[i] * sn[i] + y[i] * c[i] : y[i] * c[i] - z[i] * sn[i];
+                    if (!p.neox && e0 + i >= p.rot) r[i] = y[i];
+                }
+                y = r;
+            }
+        }
+        if (slot >= n_slot) break;
+        if (hk < 0) {
+            *reinterpret_cast<float4v*>(p.q + tok * p.tok_q + (size_t)slot * HD + e0) = y;
+        } else {
+            uint16_t* dst = (hv < 0 ? p.k_cache + (int64_t)hk * HD : p.v_cache + (int64_t)hv * HD) + rowi * p.row_stride + e0;
+            const half4 h = {(_Float16)y[0], (_Float16)y[1], (_Float16)y[2], (_Float16)y[3]};
+            *reinterpret_cast<half4*>(dst) = h;
+        }
+    }
+}
+
+// tokens per wave of the general kernel (gpt-oss 4096-token step: 1 token 34.7 us, 2 30.3, 3 30.3,
 // 4 30.0-30.8, 5 32.7, 6 33-35, 8 36.5)
 constexpr int kQkvTpw = 4;
 
@@ -177,7 +280,32 @@ hipError_t launch_qkv(const QkvParams& p, hipStream_t st) {
     auto al = [](const void* q, int a) { return (reinterpret_cast<uintptr_t>(q) % a) == 0; };
     const bool vec = al(p.q, 16) && al(p.k, 16) && al(p.v, 16) && p.tok_q % 4 == 0 && p.tok_kv % 4 == 0 &&
                      al(p.k_cache, 8) && al(p.v_cache, 8) && p.row_stride % 4 == 0;
+    // the wide kernel: 16-byte table rows and norm weights too, and a
+    // rotation whose partners are whole lanes away
+    const bool wide = vec && (!p.q_norm || al(p.q_norm, 16)) && (!p.k_norm || al(p.k_norm, 16)) &&
+                      (!p.table || (al(p.table, 16) && p.rot % (p.neox ? 8 : 4) == 0));
     ProfScope ps(kProfQkv, st);
+    if (wide) {
+        // one head group a wave while the call waits for its one round trip
+        // (gpt-oss step, ring cache: 1 token 4.5 -> 2.6 us against 3.1 with
+        // two groups and 8.5 -> 6.9 against 7.0 at 512), two once the rows'
+        // bytes bound it (4096 tokens 32.5 -> 30.1 us, 32.6 with one)
+        const int groups = (n_slot + hpw - 1) / hpw;
+        const int it = (long long)groups * p.T * p.n_seq <= 10240 ? 1 : 2;
+        const dim3 g((groups + 4 * it - 1) / (4 * it), p.T, p.n_seq);
+        auto go = [&](auto hd) {
+            constexpr int HD = decltype(hd)::value;
+            if (it == 1) hipLaunchKernelGGL((qkv_rope_cache_wide_kernel<HD, 1>), g, dim3(256), 0, st, p);
+            else hipLaunchKernelGGL((qkv_rope_cache_wide_kernel<HD, 2>), g, dim3(256), 0, st, p);
+            return hipGetLastError();
+        };
+        switch (p.hd) {
+            case 64: return go(std::integral_constant<int, 64>{});
+            case 128: return go(std::integral_constant<int, 128>{});
+            case 256: return go(std::integral_constant<int, 256>{});
+            default: return hipErrorNotSupported;
+        }
+    }
     switch (p.hd) {
         case 64: launch_hd<64>(p, vec, grid, st); break;
         case 128: launch_hd<128>(p, vec, grid, st); break;

@@ -167,3 +167,28 @@ def test_rejects_short_tables_and_odd_heads():
     with pytest.raises(attn.AttnError) as e:
         attn.qkv_rope_cache(q2, k2, v2, kc, kc.clone(), n_kv=8, kv_len=100)
     assert e.value.code == attn.EUNSUPPORTED
+
+
+@pytest.mark.parametrize("n_seq,T,n_head,n_kv,hd,rot,neox,split,norm", [
+    (1, 1, 3, 1, 64, 64, True, 0, False),      # 5 heads in a wave's 4 + 1
+    (1, 1, 1, 1, 256, 256, True, 0, True),     # one head a wave
+    (2, 5, 6, 3, 128, 24, True, 0, False),     # a rotation that ends inside a head, partners 3 lanes away
+    (2, 5, 6, 3, 128, 20, True, 0, True),      # partners half a lane away: the general kernel
+    (1, 7, 8, 2, 64, 4, False, 0, True),       # one interleaved pair of lanes
+    (1, 7, 8, 2, 64, 6, False, 0, False),      # ... that ends inside a lane: the general kernel
+    (1, 9, 4, 4, 128, 128, False, 2, True),    # two-level table, interleaved
+    (3, 260, 32, 4, 128, 128, True, 3, True),  # two head groups a wave
+    (1, 600, 63, 7, 64, 64, True, 0, False),   # ... a last group of one head
+])
+def test_wide_accesses(n_seq, T, n_head, n_kv, hd, rot, neox, split, norm):
+    L = T + 300
+    q, k, v = _case(n_seq, T, n_head, n_kv, hd, seed=T + rot)
+    if split:  # 256-position rows, then the positions within one
+        full = orc.rope_table(256 * split, rot)
+        table = torch.from_numpy(np.concatenate((full[::256], full[:256]))).cuda()
+    else:
+        table = torch.from_numpy(orc.rope_table(L, rot)).cuda()
+    w = torch.linspace(0.5, 1.5, hd, device="cuda") if norm else None
+    print(f"[case] wide T{T} h{n_head}/{n_kv} hd{hd} rot{rot} neox{neox} split{split} norm{norm}", flush=True)
+    _check(*_run_both(q, k, v, n_kv=n_kv, kv_len=L, rows=n_seq * L, table=table, rot=rot, neox=neox, table_split=split,
+                      q_norm=w, k_norm=w), "wide accesses")
