@@ -400,6 +400,8 @@ int run_decode(const PelicaAttnDesc* desc, const float* q, const uint16_t* k, co
     p.qscale = eff_scale(desc) * pelica::kLog2e;
     p.n_slot = pl.n_slot;
     p.split_keys = pl.split_keys;
+    p.inv_split = 1.0 / pl.split_keys;
+    p.hpk_mul = pelica::token_mul(p.hpk, p.R);
     p.wg_heads = pl.wg_heads;
     p.parts = parts;
     p.split_only = (desc->flags & PELICA_ATTN_FLAG_SPLIT_ONLY) != 0;
@@ -679,6 +681,8 @@ int pelica_attn_mla(const PelicaAttnDesc* desc, const float* q, const uint16_t* 
     p.qscale = eff_scale(desc) * pelica::kLog2e;
     p.n_slot = pl.n_slot;
     p.split_keys = pl.split_keys;
+    p.inv_split = 1.0 / pl.split_keys;
+    p.hpk_mul = pelica::token_mul(p.hpk, p.R);
     p.wg_heads = 1;
     p.rg_rows = 16 * pl.rt;
     hipError_t e = pelica::launch_mla(p, static_cast<hipStream_t>(stream));

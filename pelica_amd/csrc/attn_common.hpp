@@ -113,6 +113,38 @@ __device__ __forceinline__ void lds_dma16_untracked(__amdgpu_buffer_rsrc_t rsrc,
             : "s"(m), "v"(voffset), "s"(rsrc));
 }
 
+// Four such loads into 4 KB of consecutive LDS, one M0 setting for all: the
+// instruction's offset (1024 j) moves both the LDS and the memory address, so
+// load j's voffset is given without it (v[j] = its offset - 1024 j >= 0).
+template <bool NT, int J>
+__device__ __forceinline__ void lds_dma16_at(__amdgpu_buffer_rsrc_t rsrc, uint32_t v, void* lds_base) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)lds_base, 16, v, 0, 1024 * J,
+                                             NT ? 2 : 0);
+}
+template <bool NT>
+__device__ __forceinline__ void lds_dma16x4(__amdgpu_buffer_rsrc_t rsrc, const uint32_t (&v)[4], void* lds_base) {
+    lds_dma16_at<NT, 0>(rsrc, v[0], lds_base);
+    lds_dma16_at<NT, 1>(rsrc, v[1], lds_base);
+    lds_dma16_at<NT, 2>(rsrc, v[2], lds_base);
+    lds_dma16_at<NT, 3>(rsrc, v[3], lds_base);
+}
+template <bool NT>
+__device__ __forceinline__ void lds_dma16x4_untracked(__amdgpu_buffer_rsrc_t rsrc, const uint32_t (&v)[4], void* lds_base) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane(
+        (uint32_t)(size_t)(__attribute__((address_space(3))) char*)lds_base);
+    uint32_t saved;
+    static_assert(NT, "the decode stream's cache policy");
+    __asm__ volatile(
+        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+        "buffer_load_dwordx4 %2, %6, 0 offen nt lds\n\t"
+        "buffer_load_dwordx4 %3, %6, 0 offen offset:1024 nt lds\n\t"
+        "buffer_load_dwordx4 %4, %6, 0 offen offset:2048 nt lds\n\t"
+        "buffer_load_dwordx4 %5, %6, 0 offen offset:3072 nt lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "s"(m), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(rsrc));
+}
+
 // Keys of sequence s: seq_len[s] clipped to kv_len (the bound every launch
 // and workspace is sized from), or kv_len without a per-sequence table.
 __device__ __forceinline__ int seq_keys(const int32_t* seq_len, int s, int kv_len) {

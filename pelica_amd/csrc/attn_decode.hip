@@ -54,6 +54,7 @@
 // src/oss_batch.rs:172-251 (ATTN_T: window, ring, sink), :253-425 (attn_s +
 // ATTN_M: split partials, sink in max and denominator).
 #include <algorithm>
+#include <type_traits>
 
 #include "attn_decode.hpp"
 #include "attn_prof.hpp"
@@ -268,7 +269,8 @@ __device__ SkLayout sk_layout(const DecodeParams& p, int gy, const SeqTables& tb
 template <int HD, int RT, int NW, int H, bool SK>
 constexpr int kDecodeOccK = SK ? ((HD == 64 && RT == 1) ? kDecodeOcc<HD, RT, NW> : 1) : kDecodeOcc<HD, RT, NW>;
 
-template <int HD, int RT, int NW, int H, bool RING, bool PK, bool SK>
+// KQV: block 0's K, the queries, block 0's V are requested in that order
+template <int HD, int RT, int NW, int H, bool RING, bool PK, bool SK, bool KQV>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecodeOccK<HD, RT, NW, H, SK>, 8))) void decode_kernel(DecodeParams p) {
     static_assert(!SK || (H == 1 && !RING), "stream-K: one kv head per workgroup, linear caches");
     static_assert(!PK || RT == 1, "packed hi/lo columns need one row tile");
@@ -309,7 +311,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
     // then writes the output itself).  Uniform over the workgroup.
     auto split = [&](const int s, const int by, const int len, const int64_t row0, const int kbeg, const int kend,
                      const int slot, const bool single) {
-    const int kvh = (by % hgroups) * H + hl, rg = by / hgroups;
+    const int rg = p.n_rg == 1 ? 0 : by / hgroups, kvh = (by - rg * hgroups) * H + hl;
     const int lo_min = key_range(p, len, 0).lo;
     const int rbase = rg * ROWS;
 
@@ -346,49 +348,93 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
     char* vlds = klds + BUF;
     auto blk = [&](int i) { return kfirst + 64 * (wsub + W * i); };
 
-    auto row_of = [&](int i, int j) -> uint32_t {
-        const int kb = blk(i);
-        if (i >= nb) return nrec;
-        if (!RING) return (uint32_t)(kb + KPL * j + vk0 - p.kr_lo) * stride_b;
-        return (uint32_t)((kb + KPL * j + vk0) % p.ring_cap) * stride_b;
-    };
     // Load j of a block fills LDS slots j*64 + lane of the wave's buffer
     // (buffer_load ... lds).  K of a block is requested before its V, so
     // QK^T can start while V is still arriving.
     // (block 0's loads are tracked by the compiler; the loop's are
     // untracked, see the loop)
-    auto issue_k = [&](int i, bool tracked) {
+    // An offset is a lane constant (NSW of them for K: the swizzle takes
+    // 2 or 4 values) plus the block's and the load's scalar part: one vector
+    // add per load, and no multiply, branch or spilled LDS address between
+    // loads, which before stood between a small call and its last request
+    // (with the divisions of token_of / split_of: 1000-key Qwen3 decode 8.9
+    // -> 7.6 us, 2K-key OLMoE 9.7 -> 9.1, 4096-key gpt-oss 9.7 -> 9.0).
+    // Blocks past the wave's last (i >= nb) start at nrec, past every row.
+    constexpr int NSW = HD == 64 ? 2 : 4;
+    uint32_t kl[NSW];
 #pragma unroll
-        for (int j = 0; j < VPL; ++j)
-            kv_dma16(rk, row_of(i, j) + 16 * (kcol0 ^ k_swz_j<HD>(j)), klds + 1024 * j, tracked);
-    };
-    auto issue_v = [&](int i, bool tracked) {
+    for (int c = 0; c < NSW; ++c) kl[c] = (uint32_t)vk0 * stride_b + 16 * (kcol0 ^ k_swz_j<HD>(c));
+    const uint32_t vl = (uint32_t)vk0 * stride_b + vcol;
+    const uint32_t step_b = KPL * stride_b;
+    // Four loads per M0 setting, except in linear stream-K over two row
+    // tiles: its loop runs at the memory's rate with every SIMD's one wave
+    // computing beside it, and a wave stalls while a burst of four is taken
+    // (32-sequence verify 120.7 us, 122.5 with bursts).
+    constexpr bool X4 = !RING && !(SK && RT > 1);
+    auto issue = [&](const __amdgpu_buffer_rsrc_t& rs, char* lds, int i, bool is_k, bool tracked) {
+        auto lane_off = [&](int j) { return is_k ? kl[j % NSW] : vl; };
+        if constexpr (!RING) {
+            const uint32_t b = (uint32_t)uniform32(i < nb ? (int)((uint32_t)(blk(i) - p.kr_lo) * stride_b) : (int)nrec);
+            if constexpr (X4) {
+                // (step_b >= 1024: an offset less its instruction's part is >= 0)
 #pragma unroll
-        for (int j = 0; j < VPL; ++j) kv_dma16(rv, row_of(i, j) + vcol, vlds + 1024 * j, tracked);
+                for (int j = 0; j < VPL; j += 4) {
+                    uint32_t v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = lane_off(e) + (b + (j + e) * step_b - 1024 * e);
+                    if (tracked) lds_dma16x4<true>(rs, v, lds + 1024 * j);
+                    else lds_dma16x4_untracked<true>(rs, v, lds + 1024 * j);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < VPL; ++j) kv_dma16(rs, lane_off(j) + (b + j * step_b), lds + 1024 * j, tracked);
+            }
+        } else if (p.ring_cap >= 64) {
+            // the block's first row by one scalar remainder, then at most one
+            // wrap per load: the offset less the ring's bytes wherever that
+            // does not underflow (past the last block both are past the ring)
+            const uint32_t cap = (uint32_t)p.ring_cap;
+            const uint32_t b = (uint32_t)uniform32(i < nb ? (int)(((uint32_t)blk(i) % cap) * stride_b) : (int)nrec);
+            const uint32_t wrap = i < nb ? cap * stride_b : 0;
+#pragma unroll
+            for (int j = 0; j < VPL; ++j) {
+                const uint32_t o = lane_off(j) + (b + j * step_b);
+                kv_dma16(rs, min(o, o - wrap), lds + 1024 * j, tracked);
+            }
+        } else {  // (a ring shorter than a block: a remainder per load)
+#pragma unroll 1
+            for (int j = 0; j < VPL; ++j) {
+                const uint32_t row = (uint32_t)(blk(i) + KPL * j + vk0) % (uint32_t)p.ring_cap;
+                const uint32_t col = is_k ? 16 * (kcol0 ^ k_swz_j<HD>(j)) : vcol;
+                kv_dma16(rs, i < nb ? row * stride_b + col : nrec, lds + 1024 * j, tracked);
+            }
+        }
     };
+    auto issue_k = [&](int i, bool tracked) { issue(rk, klds, i, true, tracked); };
+    auto issue_v = [&](int i, bool tracked) { issue(rv, vlds, i, false, tracked); };
     // ---- block 0 and this lane's queries ----
-    // Head dim 128: the queries are requested first (a few hundred bytes
-    // per wave), then block 0 — the wait for the queries then leaves K and V
-    // in flight, so QK^T starts when K lands, not once V has (measured:
-    // 32-sequence draft batch 108.6 -> 105.3-107.0 us, 8K-key GQA decode
-    // 11.5 -> 11.3 us; the 2K-key call's split kernel 7.75 -> 7.6 us, its
-    // whole call 10.45 -> 10.6 us).
-    // Head dim 64: block 0 first, the queries behind it (the next block's K
-    // then goes out only once V has landed; requested earlier, it delays
-    // that V and the whole stream: gpt-oss decode +0.4 us, and the 128-key
-    // window call +0.7 us; with the queries first and K(1) held back until
-    // V(0) has landed, gpt-oss decode is even and the window call +0.5 us).
-    constexpr bool QFIRST = HD == 128;
-    if (!QFIRST && nb > 0) {
-        issue_k(0, true);
-        issue_v(0, true);
-    }
+    // Which of them is requested first is measured per shape, as the wait
+    // for the queries waits for what was requested before them:
+    //   K, queries, V (KQV): QK^T starts when K has landed.  Head dim 128
+    //     with one row tile (2K-key OLMoE 9.3 -> 9.05 us against queries
+    //     first); small full calls at head dim 64 (1024-4096 keys 8.4-9.3 ->
+    //     8.1-9.0 against K, V, queries).
+    //   queries, K, V: head dim 128 with two row tiles (8K-key Qwen3 verify
+    //     of one sequence 15.1 us, 15.9 with KQV).
+    //   K, V, queries: head dim 64 otherwise.  The next block's K then goes
+    //     out only once V has landed; requested earlier it delays that V
+    //     and the whole stream (32K-key gpt-oss +0.3 us; a window call, one
+    //     block a wave, +0.4 us behind the queries' address arithmetic).
+    constexpr bool QLAST = HD == 64 && !KQV;
+    if ((KQV || QLAST) && (!QLAST || nb > 0)) issue_k(0, true);
+    if (QLAST && nb > 0) issue_v(0, true);
+    __builtin_amdgcn_sched_barrier(0);  // (the requests stay in this order)
     float4v qraw[RT][DS][2];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         const int r = rbase + 16 * rt + (PK ? (c16 & 7) : c16);
         const int rr = r < p.R ? r : 0;
-        const int t = rr / p.hpk, h = kvh * p.hpk + rr % p.hpk;
+        const int t = token_of(p, rr), h = (kvh - t) * p.hpk + rr;
         const float* qp = p.q + (size_t)(s * p.T + t) * p.q_tok + h * HD + 8 * g;
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds) {
@@ -396,12 +442,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
             qraw[rt][ds][1] = *reinterpret_cast<const float4v*>(qp + 32 * ds + 4);
         }
     }
+    __builtin_amdgcn_sched_barrier(0);
     // (issued even with no block: past num_records they read zeros without
     // touching memory, and the compiler's wait for the queries is then the
     // same count on every path; such a wave waits for them before its K/V
     // buffer holds its state)
-    if (QFIRST) {
-        issue_k(0, true);
+    if (!QLAST) {
+        if (!KQV) issue_k(0, true);
         issue_v(0, true);
         if (nb == 1) DTRACE(3);  // (one-block waves: stamp 3 = block 0 requested)
     }
@@ -417,7 +464,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
         const int r = rbase + 16 * rt + (PK ? (c16 & 7) : c16);
         const bool rv_ok = r < p.R;
         const int rr = rv_ok ? r : 0;
-        const int t = rr / p.hpk;
+        const int t = token_of(p, rr);
         const KeyRange krg = key_range(p, len, t);
         posr[rt] = rv_ok ? krg.pos : -1;
         lor[rt] = krg.lo;
@@ -643,7 +690,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
             if (i + 1 < nb) issue_v(i + 1, false);
         }
     }
-    if (QFIRST && nb == 0) wait_vm<0>();  // (block 0's zero reads: the buffers hold the state next)
+    if (!QLAST && nb == 0) wait_vm<0>();  // (block 0's zero reads: the buffers hold the state next)
     DTRACE(4);
     if (PK) {
         // columns c16 and c16 ^ 8 hold the hi and lo parts of one row
@@ -719,11 +766,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
         const int r = rbase + row;
         if ((PK && c16 >= 8) || r >= p.R) continue;
         const float M = m[rt], L = l[rt];
-        const int t = r / p.hpk, h = kvh * p.hpk + r % p.hpk;
+        const int t = token_of(p, r), h = (kvh - t) * p.hpk + r;
         if (single && p.parts) {
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
-                store_part(p.parts + ((size_t)(s * p.T + t) * p.n_head + h) * (HD + 2), 16 * dt + 4 * g, M, L, o[dt][rt]);
+                store_part(p.parts + ((size_t)(s * p.T + t) * (p.n_kv * p.hpk) + h) * (HD + 2), 16 * dt + 4 * g, M, L, o[dt][rt]);
         } else if (single) {
             // the only split: normalise here, sink in max and denominator
             const float ms = (M == -INFINITY) ? 0.f : M;
@@ -768,8 +815,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
         const int len = seq_keys(p.seq_len, s, p.kv_len);
         if (len < p.T || len <= 0) return;
         const int kmax = min(len, p.kr_hi);  // keys past the last one of the call
-        const int split0 = key_range(p, len, 0).lo / p.split_keys;
-        const int n_active = min(p.n_slot, (kmax - 1) / p.split_keys - split0 + 1);
+        const int split0 = uniform32(split_of(p, key_range(p, len, 0).lo));
+        const int n_active = min(p.n_slot, uniform32(split_of(p, kmax - 1)) - split0 + 1);
         if (slot >= n_active) return;
         const int kbeg = (split0 + slot) * p.split_keys;
         const int64_t row0 = p.seq_off ? p.seq_off[s] : (int64_t)s * (p.ring_cap ? p.ring_cap : p.kv_len);
@@ -867,24 +914,26 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeParams p) {
     if (ROW_WAVES && r >= p.R) return;
     const int len = seq_keys(p.seq_len, s, p.kv_len);
     if (len < p.T || len <= 0) return;
-    const int t = r / p.hpk, h = kvh * p.hpk + r % p.hpk;
+    const int t = uniform32(token_of(p, r)), h = (kvh - t) * p.hpk + r;
     int c0, c1;  // the splits that hold keys of this row
     if (p.sk_grid > 0) {
         // stream-K: every piece of the row's segment (rows with no key in a
         // piece have an empty partial there); the split kernel records the
         // count.  (Loading every workspace slot before the count arrives was
         // measured slower: 12.6 vs 11.7 us on a 32-sequence draft batch.)
-        const int hgroups = p.n_kv / p.wg_heads;
+        // (one kv head per workgroup; several row groups are of 4 row tiles
+        // at head dim 64, of 2 at 128)
+        const int rg = p.n_rg == 1 ? 0 : r / (HD == 64 ? 64 : 32);
         c0 = 0;
-        c1 = p.ws_np[s * hgroups * p.n_rg + (r / p.rg_rows) * hgroups + kvh / p.wg_heads] - 1;
+        c1 = p.ws_np[(s * p.n_rg + rg) * p.n_kv + kvh] - 1;
         if (c1 < 1) return;  // one piece: the split kernel wrote the output
     } else {
-        const int split0 = key_range(p, len, 0).lo / p.split_keys;
-        const int n_active = min(p.n_slot, (min(len, p.kr_hi) - 1) / p.split_keys - split0 + 1);
+        const int split0 = uniform32(split_of(p, key_range(p, len, 0).lo));
+        const int n_active = min(p.n_slot, uniform32(split_of(p, min(len, p.kr_hi) - 1)) - split0 + 1);
         if (n_active <= 1) return;  // the split kernel wrote the output
         const KeyRange krg = key_range(p, len, t);
-        c0 = krg.lo / p.split_keys - split0;
-        c1 = min(krg.pos / p.split_keys - split0, n_active - 1);
+        c0 = uniform32(split_of(p, krg.lo)) - split0;
+        c1 = min(uniform32(split_of(p, krg.pos)) - split0, n_active - 1);
     }
     const size_t base = ((size_t)(s * p.n_kv + kvh) * p.R + r) * p.n_slot;
     const int ph = pt / D4, d = 4 * (pt % D4) + DW * dq;
@@ -973,7 +1022,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeParams p) {
             for (int w = 1; w < 4; ++w) merge(M, L, O, s_ml[w][tid].x, s_ml[w][tid].y, s_o[w][tid]);
         }
         if (p.parts) {
-            store_part(p.parts + ((size_t)(s * p.T + t) * p.n_head + h) * (HD + 2), d, M, L, O);
+            store_part(p.parts + ((size_t)(s * p.T + t) * (p.n_kv * p.hpk) + h) * (HD + 2), d, M, L, O);
         } else {
             // sink: in the max and the denominator
             float f = 1.f / L;
@@ -995,22 +1044,33 @@ static hipError_t launch_k(const DecodeParams& p, hipStream_t st) {
     ProfScope ps(kProfDecodeSplit, st);
     // up to 8 rows per kv head: hi and lo parts share one MFMA (packed columns)
     const bool pk = RT == 1 && p.R <= 8;
+    constexpr bool K128 = HD == 128 && RT == 1;  // (KQV: see decode_kernel)
     if (p.sk) {
+        if (p.n_rg > 1 && p.rg_rows != (HD == 64 ? 64 : 32)) return hipErrorInvalidValue;  // (the combine's row groups)
         // (the planner's stream-K shapes: 4 waves on one kv head, up to 32
         // rows per kv head at head dim 64)
         if constexpr (H == 1 && NW == 4 && !(HD == 64 && RT == 4)) {
             if (p.ring_cap || p.window || !p.seq_len) return hipErrorInvalidValue;
-            if (pk) hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, false, RT == 1, true>), dim3(p.sk_grid), dim3(64 * NW), 0, st, p);
-            else hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, false, false, true>), dim3(p.sk_grid), dim3(64 * NW), 0, st, p);
+            if (pk) hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, false, RT == 1, true, K128>), dim3(p.sk_grid), dim3(64 * NW), 0, st, p);
+            else hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, false, false, true, K128>), dim3(p.sk_grid), dim3(64 * NW), 0, st, p);
         } else {
             return hipErrorInvalidValue;
         }
     } else if (p.ring_cap) {
-        if (pk) hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, true, RT == 1, false>), grid, dim3(64 * NW), 0, st, p);
-        else hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, true, false, false>), grid, dim3(64 * NW), 0, st, p);
+        if (pk) hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, true, RT == 1, false, K128>), grid, dim3(64 * NW), 0, st, p);
+        else hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, true, false, false, K128>), grid, dim3(64 * NW), 0, st, p);
     } else {
-        if (pk) hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, false, RT == 1, false>), grid, dim3(64 * NW), 0, st, p);
-        else hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, false, false, false>), grid, dim3(64 * NW), 0, st, p);
+        auto go = [&](auto kqv) {
+            constexpr bool Q = decltype(kqv)::value;
+            if (pk) hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, false, RT == 1, false, Q>), grid, dim3(64 * NW), 0, st, p);
+            else hipLaunchKernelGGL((decode_kernel<HD, RT, NW, H, false, false, false, Q>), grid, dim3(64 * NW), 0, st, p);
+        };
+        if constexpr (HD == 64 && NW == 4) {
+            if (p.window == 0) go(std::true_type{});
+            else go(std::false_type{});
+        } else {
+            go(std::integral_constant<bool, K128>{});
+        }
     }
     }
     hipError_t e = hipGetLastError();

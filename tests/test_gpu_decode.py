@@ -321,3 +321,42 @@ def test_per_kernel_timing():
     assert names.count("decode_split") == 3 and names.count("decode_combine") == 3
     assert all(ms > 0 for _, ms in recs)
     assert attn.prof_read() == []
+
+
+@pytest.mark.parametrize("hd,n_head,n_kv,T,L,window,cap", [
+    (64, 64, 8, 1, 1000, 4, 5),        # rings shorter than a 64-key block
+    (128, 32, 4, 3, 333, 61, 63),
+    (64, 64, 8, 2, 4000, 63, 64),      # exactly one block
+    (128, 16, 16, 1, 777, 64, 65),     # blocks that wrap
+    (64, 24, 8, 4, 2500, 126, 129),
+    (128, 32, 4, 8, 5000, 900, 907),   # several blocks a wave
+    (64, 64, 8, 8, 90, 200, 207),      # a ring that has not wrapped yet
+    (64, 64, 8, 1, 300, 0, 300),       # no window: the ring holds every key
+])
+def test_ring_sizes(hd, n_head, n_kv, T, L, window, cap):
+    cfg = wl.AttnConfig("ringsz", "decode", n_head, n_kv, hd, L, q_tokens=T, window=window, sinks=True, seed=cap + T)
+    inp = wl.make_inputs(cfg, "cuda")
+    kr = torch.zeros(cap, n_kv, hd, dtype=torch.float16, device="cuda")
+    vr = torch.zeros_like(kr)
+    idx = torch.arange(max(0, L - cap), L, device="cuda")
+    kr[idx % cap] = inp.k[idx]
+    vr[idx % cap] = inp.v[idx]
+    print(f"[case] ring size hd{hd} h{n_head}/{n_kv} T{T} L{L} window{window} cap{cap}", flush=True)
+    assert_close(as_f64(gpu_run(inp, ring_cap=cap, k=kr, v=vr)), as_f64(oracle_run(inp)), what="ring size")
+
+
+@pytest.mark.parametrize("hd,n_head,n_kv,T,L,n_seq", [
+    (64, 21, 3, 1, 1500, 1),      # 7 heads per kv head
+    (64, 15, 5, 7, 700, 1),       # 21 rows: two row tiles
+    (64, 88, 8, 8, 300, 1),       # 88 rows per kv head: two groups of 64
+    (128, 40, 4, 8, 2000, 1),     # 80 rows: three groups of 32
+    (128, 40, 4, 8, 1500, 5),     # ... of a ragged batch (stream-K)
+    (64, 33, 3, 3, 900, 4),       # 33 rows: one group of 64, split grid over a ragged batch
+    (128, 13, 13, 1, 64, 1),      # one head per kv head, one block
+])
+def test_row_groups_and_odd_head_counts(hd, n_head, n_kv, T, L, n_seq):
+    cfg = wl.AttnConfig("rows", "decode", n_head, n_kv, hd, L, q_tokens=T, n_seq=n_seq, sinks=hd == 64,
+                        ragged=(T, L) if n_seq > 1 else None, seed=n_head + L)
+    inp = wl.make_inputs(cfg, "cuda")
+    print(f"[case] rows hd{hd} h{n_head}/{n_kv} T{T} L{L} n_seq{n_seq}", flush=True)
+    assert_close(as_f64(gpu_run(inp)), as_f64(oracle_run(inp)), what="row groups")
