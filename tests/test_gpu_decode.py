@@ -360,3 +360,25 @@ def test_row_groups_and_odd_head_counts(hd, n_head, n_kv, T, L, n_seq):
     inp = wl.make_inputs(cfg, "cuda")
     print(f"[case] rows hd{hd} h{n_head}/{n_kv} T{T} L{L} n_seq{n_seq}", flush=True)
     assert_close(as_f64(gpu_run(inp)), as_f64(oracle_run(inp)), what="row groups")
+
+
+def test_given_workspace_is_used_replaced_or_refused_as_before():
+    cfg = wl.AttnConfig("wsfb", "decode", 32, 4, 128, 3000, seed=9)
+    inp = wl.make_inputs(cfg, "cuda")
+    kw = dict(n_kv=4, kv_len=3000)
+    print("[case] workspace given, too small, none", flush=True)
+    ref = attn.decode(inp.q, inp.k, inp.v, **kw)
+    small = torch.zeros(16, dtype=torch.uint8, device="cuda")
+    assert torch.equal(attn.decode(inp.q, inp.k, inp.v, workspace=small, **kw), ref)  # a larger one is allocated
+    assert not small.any()
+    ws = attn.new_workspace(attn.make_desc(32, 4, 128, kv_len=3000))
+    with torch.cuda.stream(torch.cuda.Stream()):  # the current stream, not the default one
+        side = attn.decode(inp.q, inp.k, inp.v, workspace=ws, **kw)
+        torch.cuda.current_stream().synchronize()
+    assert torch.equal(side, ref)
+    with pytest.raises(AssertionError):
+        attn.decode(inp.q, inp.k, inp.v, workspace=ws, sinks=torch.zeros(5, device="cuda"), **kw)
+    for bad in (dict(window=-1), dict(kv_row_stride=8), dict(kv_len=0)):
+        with pytest.raises(attn.AttnError) as e:
+            attn.decode(inp.q, inp.k, inp.v, workspace=ws, **{**kw, **bad})
+        assert e.value.code == attn.EINVAL
