@@ -25,7 +25,6 @@
 // one kv head (its K/V stays in that XCD's L2) and the longest key ranges
 // start first.
 #include <algorithm>
-#include <cstdlib>
 #include <type_traits>
 
 #include "attn_prefill.hpp"
@@ -77,9 +76,10 @@ __device__ __forceinline__ int v_slot(int k, int p) {
 }
 
 // waves per SIMD: 2 (64 query rows per wave at hd 64, 32 at hd 128), or 1
-// with 128 rows per wave (the whole register file for one wave)
-template <int HD, int RT>
-constexpr int kPrefillOcc = HD * RT >= 256 ? 1 : 2;
+// with 128 rows per wave (the whole register file for one wave) or where four
+// one-wave key groups fill the LDS
+template <int HD, int RT, int NW, int KG>
+constexpr int kPrefillOcc = HD * RT >= 256 || (NW == 4 && KG > 1) ? 1 : 2;
 
 // Build-time instrumentation (off by default; -DPELICA_PTRACE): per wave,
 // shader-clock cycles spent in the tile loop, waiting for tile loads and at
@@ -105,7 +105,7 @@ __device__ __forceinline__ unsigned long long rtime() { return __builtin_amdgcn_
 // buffers, TK keys a tile (64, or 32 where LDS holds no more); the groups'
 // (m, l, O) states are merged through LDS after the last chunk.
 template <int HD, int RT, bool RING, bool ROUND, int NW, int NRES = 0, bool F32 = false, int KG = 1, int TK = 64>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefillOcc<HD, RT>, kPrefillOcc<HD, RT>))) void prefill_kernel(
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefillOcc<HD, RT, NW, KG>, kPrefillOcc<HD, RT, NW, KG>))) void prefill_kernel(
     PrefillParams p, int n_tb, int TB) {
     constexpr int KS = HD / 16;                 // 16-dim k-steps of QK^T
     constexpr int DT = HD / 32;                 // 32-dim output tiles
@@ -1339,11 +1339,12 @@ static int prefill_cus() {
 // How an 8-wave launch cuts its work: `split` 1 is one key group per
 // workgroup on all of its rows; each step halves a workgroup's rows and
 // doubles the number of workgroups: key groups 2, 4 and (head dim 64) 8, then
-// (16) eight groups with one row tile a wave.  Few rows leave most CUs idle
+// (16) eight groups with one row tile a wave; at head dim 128 the last (8) is
+// four groups of one wave, as LDS holds no more.  Few rows leave most CUs idle
 // otherwise: 512 gpt-oss tokens are 64 workgroups of 512 rows, and a full
 // layer at position 30K took 772 us with 1 group, 414 with 2, 278 with 4, 317
 // with 8 (512 workgroups: two generations); 256 Qwen3 tokens over 27K keys
-// (two rounds) 635 / 331 / 224; 64 gpt-oss tokens at 8K 204 / 110 / 62 / 40 /
+// (two rounds) 635 / 331 / 224 / 206; 64 gpt-oss tokens at 8K 204 / 110 / 62 / 40 /
 // 27.5.  Where the grid fills the chip anyway, groups only cost: each loads
 // its own keys (LDS writes beside the operand reads), and every workgroup
 // pays its start and its merge (4096 fresh gpt-oss tokens 147 / 164 / 205 /
@@ -1356,14 +1357,12 @@ struct SplitCost {
 };
 constexpr SplitCost kSplitCost64[5] = {{.0244f, 3.5f, .0325f, 4.0f}, {.0246f, 5.5f, .0330f, 6.8f}, {.0285f, 6.0f, .0350f, 8.0f},
                                        {.0300f, 6.0f, .0370f, 8.0f}, {.0250f, 3.0f, .0250f, 4.8f}};
-constexpr SplitCost kSplitCost128[3] = {{.0232f, 4.0f, .0375f, 4.0f}, {.0240f, 5.0f, .0385f, 7.0f}, {.0325f, 5.0f, .0407f, 8.0f}};
+constexpr SplitCost kSplitCost128[4] = {{.0232f, 4.0f, .0375f, 4.0f}, {.0240f, 5.0f, .0385f, 7.0f}, {.0325f, 5.0f, .0407f, 8.0f},
+                                        {.0290f, 4.2f, .0270f, 5.0f}};
 
 static int prefill_split(const PrefillParams& p, int rows) {
-#ifdef KG_ENV
-    if (const char* e = getenv("PELICA_KG")) return atoi(e);
-#endif
     const SplitCost* const cost = p.hd == 64 ? kSplitCost64 : kSplitCost128;
-    const int n_split = p.hd == 64 ? 5 : 3;
+    const int n_split = p.hd == 64 ? 5 : 4;
     const double cus = prefill_cus();
     // keys of the longest token block, and how many fewer the shortest walks
     const double keys = p.state ? p.key_end - p.key_begin : p.kv_len;
@@ -1374,7 +1373,7 @@ static int prefill_split(const PrefillParams& p, int rows) {
     double best = 0;
     int pick = 1;
     for (int i = 0; i < n_split; ++i) {
-        const int split = 1 << i, TB = rows / split / p.hpk, kg = std::min(split, 8);
+        const int split = 1 << i, TB = rows / split / p.hpk, kg = std::min(split, p.hd == 64 ? 8 : 4);
         if (TB == 0 || (i > 0 && !fits)) break;
         const long long n_tb = (p.T + TB - 1) / TB, n = n_tb * same;
         auto walk = [&](long long b) { return (keys - (double)(b / same) / n_tb * spread) / kg; };  // block b, longest first
@@ -1397,7 +1396,7 @@ template <int HD, int RT, int NW, bool F32>
 static hipError_t launch_nw(const PrefillParams& p, hipStream_t st) {
     constexpr int ROWS = NW * RT * 32;
     if (p.hpk > ROWS) return hipErrorNotSupported;
-    const int split = NW == 8 && !p.ring_cap ? prefill_split(p, ROWS) : 1, KG = std::min(split, 8);
+    const int split = NW == 8 && !p.ring_cap ? prefill_split(p, ROWS) : 1, KG = std::min(split, HD == 64 ? 8 : 4);
     const int TB = ROWS / split / p.hpk;
     const int n_tb = (p.T + TB - 1) / TB;
     const long long nblk = (long long)n_tb * p.n_kv * p.n_seq;
@@ -1425,6 +1424,14 @@ static hipError_t launch_nw(const PrefillParams& p, hipStream_t st) {
             };
             using std::integral_constant;
             using RTc = integral_constant<int, RT>;
+            if constexpr (HD == 128) {
+                if (split == 8) {  // (four one-wave groups)
+                    const dim3 b4(256);
+                    if (p.state) hipLaunchKernelGGL((prefill_kernel<HD, 1, false, true, 4, 0, F32, 4, 32>), grid, b4, 0, st, p, n_tb, TB);
+                    else hipLaunchKernelGGL((prefill_kernel<HD, 1, false, false, 4, 0, F32, 4, 32>), grid, b4, 0, st, p, n_tb, TB);
+                    return hipGetLastError();
+                }
+            }
             if (KG == 2) go(RTc{}, integral_constant<int, 2>{}, integral_constant<int, 64>{});
             else if (KG == 4) go(RTc{}, integral_constant<int, 4>{}, integral_constant<int, TK4>{});
             else if constexpr (HD == 64) {

@@ -195,8 +195,10 @@ def test_slide_window_ring_ragged_sequences():
     (64, 64, 8, 700, 700, 2, None, 0),      # two
     (64, 64, 8, 5, 5, 1, None, 0),          # one chunk: every group but the first walks nothing
     (64, 64, 8, 100, 3000, 1, None, 1500),  # a window too long for the short-window kernels
-    (128, 32, 4, 256, 256, 1, None, 0),     # head dim 128: four groups of 32-key tiles
+    (128, 32, 4, 256, 256, 1, None, 0),     # head dim 128: four one-wave groups
     (128, 16, 16, 33, 2049, 1, None, 0),    # ... an odd share of the chunks
+    (128, 40, 1, 9, 600, 1, None, 0),       # ... whose 32 rows hold no token of 40 heads
+    (128, 32, 4, 500, 520, 1, None, 0),     # four two-wave groups of 32-key tiles
     (128, 32, 4, 1000, 1000, 1, None, 0),   # two groups
     (128, 32, 4, 40, 3000, 3, (40, 3000), 0),   # ragged: short sequences leave whole groups without keys
 ])
@@ -216,6 +218,7 @@ def test_key_groups(hd, n_head, n_kv, T, L, n_seq, ragged, window, f32):
     (64, 64, 8, 40, 3000, [0, 1, 700, 2980, 3000], 0),   # a last round that only some tokens see
     (64, 64, 8, 250, 6000, [0, 5000, 5800, 6000], 0),
     (128, 32, 4, 100, 5000, [0, 777, 3000, 5000], 0),
+    (128, 32, 4, 490, 2000, [0, 1000, 1510, 2000], 0),
     (64, 64, 8, 64, 4000, [0, 1500, 4000], 1600),
 ])
 def test_key_groups_in_rounds(hd, n_head, n_kv, T, L, bounds, window):
