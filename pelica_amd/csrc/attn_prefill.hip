@@ -6,7 +6,9 @@
 // of that kv head's GQA group, so each K/V tile staged in LDS serves every
 // head of the group.  Each wave holds RT tiles of 32 rows.  Keys stream in
 // 64-key tiles, double-buffered in LDS: the next tile's global loads are in
-// flight while the current one is computed.
+// flight while the current one is computed.  Where the rows are too few for
+// the chip, a workgroup's waves form key groups over the same rows and merge
+// their states at the end (prefill_split).
 //
 // Per tile and wave, on v_mfma_f32_32x32x16_f16:
 //   S^T[key][row] = K Q^T — K read from LDS (ds_read_b128, XOR-swizzled rows)
@@ -1450,10 +1452,6 @@ static hipError_t launch_nw(const PrefillParams& p, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Workgroup size: 8 waves (2 per SIMD from one workgroup: each K/V tile in
-// LDS serves twice the rows; the 4096-token gpt-oss causal prefill ~2 %
-// faster) unless a short window makes the larger token block mostly masked
-// (window 128: 4 waves, 25 % faster than 8).
 // ring slots of the sliding-window kernel: the chunks of two consecutive
 // 64-token blocks, (126 + window) / 32 + 2, fit for windows up to 130
 constexpr int kSlideChunks = 10;
@@ -1482,6 +1480,10 @@ static hipError_t launch_slide(const PrefillParams& p, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Workgroup size: 8 waves (2 per SIMD from one workgroup: each K/V tile in
+// LDS serves twice the rows; the 4096-token gpt-oss causal prefill ~2 %
+// faster) unless a short window makes the larger token block mostly masked
+// (window 128: 4 waves, 25 % faster than 8).
 template <int HD, int RT, bool F32>
 static hipError_t launch(const PrefillParams& p, hipStream_t st) {
     if constexpr (HD == 64) {
