@@ -171,11 +171,6 @@ int plan_decode(const PelicaAttnDesc* d, DecodePlan* pl, int kr_len = 0) {
     // keys any row of a sequence can see
     const long long span = d->window > 0 ? std::min<long long>(d->kv_len, (long long)d->window + d->q_tokens - 1)
                                          : d->kv_len;
-    // A key range plans the splits of the whole cache (the same split size,
-    // so its workspace is never larger than pelica_attn_workspace_bytes
-    // gives) and keeps the splits that hold its keys.
-    const long long span_r = kr_len > 0 ? std::min<long long>(span, kr_len) : span;
-    const bool bounded = d->window > 0 || kr_len > 0;
     const long long groups = (long long)d->n_seq * d->n_kv * n_rg;
     const long long blocks = (long long)ceil_div(span, 64) * groups;
     // Workgroup shape.  Large head-dim-64 calls: 8 waves, 4 kv heads per
@@ -199,40 +194,52 @@ int plan_decode(const PelicaAttnDesc* d, DecodePlan* pl, int kr_len = 0) {
     const int target_waves = std::max(64, tn.decode_waves ? tn.decode_waves : (big ? 2048 : 1024));
     int spw = tn.split_blocks;
     if (spw <= 0) spw = (int)std::max<long long>(1, (blocks + target_waves - 1) / target_waves);
-    auto splits = [&](int nw_, long long* keys, int* ns) {
-        long long split_keys = 64LL * (nw_ / wg_heads) * spw;
-        int n_slot = 0;
-        for (;;) {
-            const int total = ceil_div(d->kv_len, split_keys);
-            n_slot = bounded ? std::min<int>(total, ceil_div(span_r, split_keys) + 1) : total;
-            if (n_slot <= pelica::kMaxSlots) break;
-            split_keys *= 2;
+    int nw = 0, n_slot = 0;
+    long long split_keys = 0;
+    // the split of `seen` keys (bounded: of a longer cache)
+    auto choose = [&](long long seen, bool bounded) {
+        auto splits = [&](int nw_) {
+            nw = nw_;
+            split_keys = 64LL * (nw / wg_heads) * spw;
+            for (;;) {
+                const int total = ceil_div(d->kv_len, split_keys);
+                n_slot = bounded ? std::min<int>(total, ceil_div(seen, split_keys) + 1) : total;
+                if (n_slot <= pelica::kMaxSlots) break;
+                split_keys *= 2;
+            }
+        };
+        splits(big ? 8 : 4);
+        // Small head-dim-128 calls: with 4-wave workgroups the grid would not
+        // reach every CU (a CU pulls ~22 GB/s at most here), so split the keys
+        // four times as finely over one-wave workgroups: every wave writes its
+        // own split's partials, with no merge between waves after its last
+        // block (OLMoE 2K / Qwen3 8K decode: split kernel 7.45 -> 6.97 /
+        // 7.68 -> 6.88 us against 2-wave workgroups, whole call 10.14 -> 9.95
+        // / 10.87 -> 10.45 us).
+        if (!big && d->hd == 128 && (long long)n_slot * groups < device_cus()) splits(1);
+        // Window layers: when the keys any row sees fit one workgroup (each wave
+        // <= 2 blocks), one split per kv head — the workgroup merges its waves
+        // and writes the output itself, no combine launch.
+        if (d->window > 0 && !big && (ceil_div(span, 64) + 1) <= 2 * (nw / wg_heads) && tn.split_blocks == 0) {
+            split_keys = ((long long)d->kv_len + 63) / 64 * 64;
+            n_slot = 1;
         }
-        *keys = split_keys;
-        *ns = n_slot;
     };
-    int nw = big ? 8 : 4;
-    long long split_keys;
-    int n_slot;
-    splits(nw, &split_keys, &n_slot);
-    // Small head-dim-128 calls: with 4-wave workgroups the grid would not
-    // reach every CU (a CU pulls ~22 GB/s at most here), so split the keys
-    // four times as finely over one-wave workgroups: every wave writes its
-    // own split's partials, with no merge between waves after its last
-    // block (OLMoE 2K / Qwen3 8K decode: split kernel 7.45 -> 6.97 /
-    // 7.68 -> 6.88 us against 2-wave workgroups, whole call 10.14 -> 9.95
-    // / 10.87 -> 10.45 us).
-    if (!big && d->hd == 128 && (long long)n_slot * groups < device_cus()) {
-        nw = 1;
-        splits(nw, &split_keys, &n_slot);
-    }
-    // Window layers: when the keys any row sees fit one workgroup (each wave
-    // <= 2 blocks), one split per kv head — the workgroup merges its waves
-    // and writes the output itself, no combine launch.
-    if (d->window > 0 && !big && (ceil_div(span, 64) + 1) <= 2 * (nw / wg_heads) &&
-        tn.split_blocks == 0) {
-        split_keys = ((long long)d->kv_len + 63) / 64 * 64;
-        n_slot = 1;
+    choose(span, d->window > 0);
+    if (kr_len > 0) {
+        // A key range takes its own split where the whole cache's workspace
+        // (pelica_attn_workspace_bytes, which knows no range) holds it, else
+        // the splits of the whole cache that hold its keys: few of them may
+        // otherwise turn to one-wave workgroups with more slots than the
+        // whole cache has.
+        const long long span_r = std::min<long long>(span, kr_len), keys_all = split_keys;
+        const int slots_all = n_slot, nw_all = nw;
+        choose(span_r, true);
+        if (n_slot > slots_all) {
+            nw = nw_all;
+            split_keys = keys_all;
+            n_slot = std::min(slots_all, ceil_div(span_r, split_keys) + 1);
+        }
     }
     pl->sk = sk;
     pl->sk_grid = pl->sk_minb = pl->sk_restart = 0;

@@ -250,6 +250,41 @@ def test_key_range_arguments():
     assert b"one sequence" in lib.pelica_attn_last_error()
 
 
+def test_key_range_fits_the_documented_workspace():
+    # any range of a cache runs in the workspace of the whole cache's decode:
+    # asked with one byte of workspace, the call says what it needs (a range
+    # of one split needs none and would launch: without a GPU, an error)
+    import random
+    import re
+
+    import torch
+
+    if torch.cuda.device_count():
+        pytest.skip("the pointers are stand-ins: for machines without a GPU")
+    lib = attn.load_library()
+    rng = random.Random(3)
+    cases = [(16, 16, 128, 4, 19455, 3635, 18537, 0), (40, 4, 128, 3, 16145, 10673, 16106, 0),
+             (32, 4, 128, 8, 8000, 0, 6000, 0), (16, 16, 128, 1, 12230, 4134, 10356, 0)]
+    for _ in range(4000):
+        H, G, hd = rng.choice([(64, 8, 64), (32, 4, 128), (16, 16, 128), (40, 4, 128), (24, 8, 64)])
+        T = rng.choice([1, 2, 3, 4, 8])
+        L = rng.randint(T, rng.choice([2000, 20000, 200000]))
+        a = rng.randrange(L)
+        cases.append((H, G, hd, T, L, a, rng.randint(a + 1, L), rng.choice([0, 0, 128, 1000])))
+    checked = 0
+    for H, G, hd, T, L, a, b, window in cases:
+        d = ctypes.byref(attn.make_desc(H, G, hd, q_tokens=T, kv_len=L, window=window))
+        whole = lib.pelica_attn_workspace_bytes(d)
+        if whole == 0:  # (one split: such a call would launch)
+            continue
+        rc = lib.pelica_attn_decode_partials_range(d, 16, 16, 16, a, b, 16, 16, 1, None)
+        if rc == attn.EWORKSPACE:
+            need = int(re.match(rb"workspace of (\d+) bytes", lib.pelica_attn_last_error()).group(1))
+            assert need <= whole, (H, G, hd, T, L, a, b, window)
+            checked += 1
+    assert checked > 2000
+
+
 def test_recorded_traffic_follows_the_kernel_sources(tmp_path, monkeypatch):
     # bench.py reports roofline.traffic from the committed counter summary
     # only while the kernel's sources hash as they did when it was measured
