@@ -33,8 +33,8 @@ F16_PEAK_TFLOPS = 2500.0    # MI355X dense f16 MFMA
 # whose sources have changed since is not reported.
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "hbm_traffic_counters.md")
 KERNEL_SOURCES = {
-    "decode": ("attn_decode.hip", "attn_decode.hpp", "attn_common.hpp"),
-    "prefill": ("attn_prefill.hip", "attn_prefill.hpp", "attn_common.hpp"),
+    "decode": ("attn_decode.hip", "attn_decode.hpp", "attn_plan.hpp", "attn_common.hpp"),
+    "prefill": ("attn_prefill.hip", "attn_prefill.hpp", "attn_plan.hpp", "attn_common.hpp"),
 }
 # rocprofv3 kernel-name prefix and source set of each config's dominant kernel
 TRAFFIC_KERNELS = {

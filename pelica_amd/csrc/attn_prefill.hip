@@ -162,6 +162,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     const int kbeg = ROUND ? p.key_begin : 0, kend = ROUND ? min(p.key_end, len) : len;
     const uint32_t stride_b = (uint32_t)p.row_stride * 2;
     const int klast = min(pos_last, kend - 1);  // the last key a row sees
+    // every row sees every key from lo_all to hi_all of this launch
+    const int lo_all = ROUND ? max(lo_last, kbeg) : lo_last, hi_all = ROUND ? min(pos_first, kend - 1) : pos_first;
     // (key groups: rows past klast, in a share's tail, read as zeros too)
     const uint32_t nrec = (RING ? (uint32_t)p.ring_cap : (uint32_t)max(0, (KG > 1 ? klast + 1 : kend) - kbeg)) * stride_b;
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
@@ -270,6 +272,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         }
         posr[rt] = valid[rt] ? len - p.T + t : -1;
         lor[rt] = (p.window > 0 && posr[rt] + 1 > p.window) ? posr[rt] + 1 - p.window : 0;
+        // (of this round's keys; one bound each side, as the loop has no
+        // scalar registers to spare: 256 Qwen3 tokens over 27K keys in two
+        // rounds 212 us with the round's own bounds beside these, 199 so)
+        if (ROUND) {
+            posr[rt] = min(posr[rt], kend - 1);
+            lor[rt] = max(lor[rt], kbeg);
+        }
     }
 
     // running state; a sink starts it at (max = sink, sum = 1)
@@ -406,11 +415,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         // per 32-key chunk, one group / four groups: head dim 64 1966 / 2490
         // -> 1900 / 2064, head dim 128 1826 / 2400 -> 1722 / 2100).  No
         // branches there either (they cost more than the burst): a tile past
-        // the last one is requested past the rows, which reads nothing.
+        // the last one is requested past the rows (tile_base), which reads
+        // nothing.
         constexpr int NLD = SPREAD && (CPT == 1 || (PAR & 1)) ? 2 * WI : 0;
         const int tk = t + 2, tv = t + CPT - 1;
-        const uint32_t off_k = tk < n_tiles ? (uint32_t)(kb0 + TK * tk - kbeg) * stride_b : 0xF0000000u;
-        const uint32_t off_v = tv < n_tiles ? (uint32_t)(kb0 + TK * tv - kbeg) * stride_b : 0xF0000000u;
+        const uint32_t off_k = tile_base(tk < n_tiles, kb0 + TK * tk - kbeg, stride_b);
+        const uint32_t off_v = tile_base(tv < n_tiles, kb0 + TK * tv - kbeg, stride_b);
         auto load_nth = [&](int n) {
             const bool is_v = n >= WI;
             const int i = is_v ? n - WI : n, slot = 64 * (NWG * i + wr) + lane, key = slot / PPR, phys = slot % PPR;
@@ -420,14 +430,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
         };
 
         const int kb = kb0 + 32 * c;
-        if (kb + 31 > pos_first || kb < lo_last || (ROUND && (kb < kbeg || kb + 31 >= kend))) {
+        if (kb + 31 > hi_all || kb < lo_all) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int key = kb + 8 * (i / 4) + 4 * h2 + (i % 4);
-                const bool out_of_round = ROUND && (key < kbeg || key >= kend);
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt)
-                    if (key < lor[rt] || key > posr[rt] || out_of_round) s_cur[rt][i] = -INFINITY;
+                    if (key < lor[rt] || key > posr[rt]) s_cur[rt][i] = -INFINITY;
             }
         }
 

@@ -1,6 +1,7 @@
 // Launch parameters of the prefill kernel (attn_prefill.hip).
 #pragma once
 #include "attn_common.hpp"
+#include "attn_plan.hpp"
 
 namespace pelica {
 
