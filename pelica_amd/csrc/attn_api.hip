@@ -391,9 +391,12 @@ int run_decode(const PelicaAttnDesc* desc, const float* q, const uint16_t* k, co
     p.row_stride = desc->kv_row_stride ? desc->kv_row_stride : (int64_t)desc->n_kv * desc->hd;
     p.q_tok = q_stride(desc);
     p.o_tok = o_stride(desc);
-    p.kr_lo = key_end > 0 ? key_begin : 0;
-    p.kr_hi = key_end > 0 ? key_end : INT32_MAX;
-    p.kv_len = desc->kv_len;
+    // (a key range: all positions moved up to where its keys begin a split;
+    // they count from there in every use)
+    const int shift = key_end > 0 ? pelica::range_shift(key_begin, pl.split_keys) : 0;
+    p.kr_lo = key_end > 0 ? key_begin + shift : 0;
+    p.kr_hi = key_end > 0 ? key_end + shift : INT32_MAX;
+    p.kv_len = desc->kv_len + shift;
     p.n_head = desc->n_head;
     p.n_kv = desc->n_kv;
     p.hd = desc->hd;

@@ -323,8 +323,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
     // Buffer resources over this sequence's rows of kv head kvh: 32-bit
     // offsets, and loads at offsets past num_records return 0 without
     // touching memory — the tail of the last block costs no traffic.  (A
-    // key range's rows start at position kr_lo: keys below it wrap to
-    // offsets past num_records.)
+    // key range's rows start at position kr_lo, the first of a split: no
+    // block starts below it.)
     const uint32_t stride_b = (uint32_t)p.row_stride * 2;
     const uint32_t nrec = (RING ? (uint32_t)p.ring_cap : (uint32_t)(min(len, p.kr_hi) - p.kr_lo)) * stride_b;
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
@@ -379,12 +379,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
         if constexpr (!RING) {
             const uint32_t b = (uint32_t)uniform32(i < nb ? (int)((uint32_t)(blk(i) - p.kr_lo) * stride_b) : (int)nrec);
             if constexpr (X4) {
-                // (step_b >= 1024: an offset less its instruction's part is >= 0)
 #pragma unroll
                 for (int j = 0; j < VPL; j += 4) {
                     uint32_t v[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = lane_off(e) + (b + (j + e) * step_b - 1024 * e);
+                    for (int e = 0; e < 4; ++e) v[e] = burst_offset(lane_off(e), b, step_b, j, e);
                     if (tracked) lds_dma16x4<true>(rs, v, lds + 1024 * j);
                     else lds_dma16x4_untracked<true>(rs, v, lds + 1024 * j);
                 }

@@ -1,6 +1,7 @@
 // Launch parameters of the decode kernel (attn_decode.hip).
 #pragma once
 #include "attn_common.hpp"
+#include "attn_plan.hpp"
 
 namespace pelica {
 
@@ -30,7 +31,7 @@ struct DecodeParams {
     int64_t row_stride;  // f16 values between cache rows
     int64_t q_tok, o_tok;  // f32 values between consecutive query / output tokens
     int kr_lo, kr_hi;    // the call's key positions [kr_lo, kr_hi) (0, INT32_MAX: all);
-                         // cache row 0 holds position kr_lo
+                         // cache row 0 holds position kr_lo, a multiple of split_keys
     int kv_len, n_kv, hpk, T, R, n_seq, n_rg;
     uint32_t hpk_mul;    // token_of's multiplier, 0: divide
     int window, ring_cap;

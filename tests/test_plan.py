@@ -18,6 +18,9 @@ def plan(tmp_path_factory):
     u32, i32 = ctypes.c_uint32, ctypes.c_int32
     lib.tile_base.restype = u32
     lib.tile_base.argtypes = [i32, i32, u32]
+    lib.range_shift.argtypes = [i32, i32]
+    lib.burst_offset.restype = u32
+    lib.burst_offset.argtypes = [u32, u32, u32, i32, i32]
     return lib
 
 
@@ -51,3 +54,29 @@ def test_wanted_tile_starts_at_its_row(plan):
     for rows, stride in _spans():
         for first in {0, rows // 2, rows - 1}:
             assert plan.tile_base(1, first, stride) == first * stride
+
+
+def test_key_range_blocks_start_at_its_rows(plan):
+    # every 64-key block of a range starts at one of its rows or past them, so
+    # no row's offset, less the instruction's own part, falls below zero; and
+    # the range lies in as few splits as its keys fill
+    rng = random.Random(2)
+    for _ in range(3000):
+        split = 64 * rng.choice((1, 1, 2, 3, 4, 7, 16, 100))
+        begin = rng.randrange(40000)
+        keys = rng.randint(1, 9000)
+        shift = plan.range_shift(begin, split)
+        lo = begin + shift  # the position of row 0
+        assert 0 <= shift < split
+        first_split, last_split = lo // split, (lo + keys - 1) // split
+        assert last_split - first_split + 1 == -(-keys // split)
+        hd = rng.choice((64, 128))
+        per_load, stride = 512 // hd, hd * 2 * rng.choice((1, 4, 8, 32, 4096))
+        first = first_split * split - lo  # the first block's row
+        b = first * stride % (1 << 32)
+        j, e, lane = 4 * rng.randrange(hd // 32), rng.randrange(4), rng.randrange(64)
+        lane_off = lane // (hd // 8) * stride + lane % (hd // 8) * 16
+        row = first + per_load * (j + e) + lane // (hd // 8)
+        assert row >= 0
+        off = plan.burst_offset(lane_off, b, per_load * stride, j, e)
+        assert off + 1024 * e == row * stride + lane % (hd // 8) * 16
