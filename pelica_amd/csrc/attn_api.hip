@@ -366,6 +366,14 @@ int run_decode(const PelicaAttnDesc* desc, const float* q, const uint16_t* k, co
     DecodePlan pl;
     int rc = plan_decode(desc, &pl, key_end > 0 ? key_end - key_begin : 0);
     if (rc) return rc;
+    if (key_end > 0 && desc->window > 0 && desc->kv_len - desc->q_tokens + 1 - desc->window >= key_end) {
+        // every row's window begins past the range: one split, whose
+        // workgroups write the empty slots (of several, none would hold a
+        // key that a row sees, and none would write)
+        pl.n_slot = 1;
+        pl.split_keys = ceil_div(desc->kv_len, 64) * 64;
+        pl.ws_bytes = 0;
+    }
     rc = check_strides(desc, 4, 4);
     if (rc) return rc;
     if (!q || !k || !v || !(out || parts))

@@ -150,6 +150,25 @@ def test_key_range_slots_of_rows_that_see_none_of_it():
     assert np.all(p[..., 0] <= -1e38) and np.all(p[..., 1:] == 0)
 
 
+@pytest.mark.parametrize("H,G,hd,T,L,window,a,b", [
+    (64, 8, 64, 1, 30000, 2000, 0, 10000),       # the range ends many splits before any window begins
+    (64, 8, 64, 4, 30000, 2000, 300, 27997),     # ... at the key before the first window
+    (32, 4, 128, 8, 20000, 1500, 1000, 9000),
+    (16, 16, 128, 1, 12000, 4000, 0, 1),
+])
+def test_key_range_before_every_long_window(H, G, hd, T, L, window, a, b):
+    # windows over several splits: every slot is written, and empty
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q = torch.randn(1, T, H, hd, device="cuda", generator=g)
+    k = torch.randn(b - a, G, hd, device="cuda", generator=g).half()
+    parts = torch.full((1, T, H, hd + 2), float("nan"), device="cuda")
+    print(f"[case] range [{a}, {b}) of {L} before every window of {window}, h{H}/{G} hd{hd} T{T}", flush=True)
+    attn.decode_partials_range(q, k, k.clone(), n_kv=G, kv_len=L, key_begin=a, key_end=b, window=window, parts=parts)
+    torch.cuda.synchronize()
+    p = parts.cpu().numpy()
+    assert np.all(p[..., 0] <= -1e38) and np.all(p[..., 1:] == 0)
+
+
 def test_f32_prefill_rounds_over_staged_rows():
     # attn_p's far rows come from a staging copy: rounds [0, res) and [res, L)
     T, L, res = 300, 700, 450
