@@ -168,13 +168,15 @@ __global__ __launch_bounds__(256) void qkv_rope_cache_kernel(QkvParams p) {
 // and a rotation partner comes from its lane's registers, not through LDS.
 // Small steps are one dependent chain of load, exchange and store: fewer
 // instructions and more waves shorten it; large ones run at the copy rate.
-template <int HD, int IT>
+// TPB tokens a workgroup, 4 / TPB of its waves along the heads (launch_qkv).
+template <int HD, int IT, int TPB>
 __global__ __launch_bounds__(256) void qkv_rope_cache_wide_kernel(QkvParams p) {
-    constexpr int LPH = HD / 4, HPW = 64 / LPH;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane / LPH, e0 = 4 * (lane % LPH);
-    const int t = blockIdx.y, s = blockIdx.z, n_slot = p.n_head + 2 * p.n_kv;
-    const int slot0 = (blockIdx.x * 4 + wave) * (HPW * IT) + sub;
-    if (slot0 - sub >= n_slot) return;
+    constexpr int LPH = HD / 4, HPW = 64 / LPH, WX = 4 / TPB;
+    const int wave = TPB > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, sub = lane / LPH, e0 = 4 * (lane % LPH);
+    const int t = blockIdx.y * TPB + (TPB > 1 ? wave / WX : 0), s = blockIdx.z, n_slot = p.n_head + 2 * p.n_kv;
+    const int slot0 = (blockIdx.x * WX + (TPB > 1 ? wave % WX : wave)) * (HPW * IT) + sub;
+    if (slot0 - sub >= n_slot || (TPB > 1 && t >= p.T)) return;
     const int len = seq_keys(p.seq_len, s, p.kv_len);
     if (len < p.T || len > p.kv_len) return;  // (attention skips such sequences too)
     const size_t tok = (size_t)s * p.T + t;
@@ -292,11 +294,23 @@ hipError_t launch_qkv(const QkvParams& p, hipStream_t st) {
         // bytes bound it (4096 tokens 32.5 -> 30.1 us, 32.6 with one)
         const int groups = (n_slot + hpw - 1) / hpw;
         const int it = (long long)groups * p.T * p.n_seq <= 10240 ? 1 : 2;
-        const dim3 g((groups + 4 * it - 1) / (4 * it), p.T, p.n_seq);
+        const int waves = (groups + it - 1) / it;  // of one token
+        // Workgroups go round the 8 XCDs in order: with an even number of
+        // them along the heads, a last one with idle waves falls to the same
+        // XCDs for every token.  The least tokens a workgroup (4, 2 or 1
+        // waves along the heads) that leaves none idle, or an odd number
+        // (4096 tokens: 24 + 16 heads of 64 19.0 -> 15.7 us, 40 + 16 of 128
+        // with norms 42.0 -> 38.5; two tokens where the number is odd already
+        // only cost: 64 + 16 of 64 27.0 -> 27.5).
+        int tpb = 1;
+        while (it == 2 && tpb < 4 && waves % (4 / tpb) != 0 && (waves + 4 / tpb - 1) / (4 / tpb) % 2 == 0) tpb *= 2;
+        const dim3 g((waves + 4 / tpb - 1) / (4 / tpb), (p.T + tpb - 1) / tpb, p.n_seq);
         auto go = [&](auto hd) {
             constexpr int HD = decltype(hd)::value;
-            if (it == 1) hipLaunchKernelGGL((qkv_rope_cache_wide_kernel<HD, 1>), g, dim3(256), 0, st, p);
-            else hipLaunchKernelGGL((qkv_rope_cache_wide_kernel<HD, 2>), g, dim3(256), 0, st, p);
+            if (it == 1) hipLaunchKernelGGL((qkv_rope_cache_wide_kernel<HD, 1, 1>), g, dim3(256), 0, st, p);
+            else if (tpb == 1) hipLaunchKernelGGL((qkv_rope_cache_wide_kernel<HD, 2, 1>), g, dim3(256), 0, st, p);
+            else if (tpb == 2) hipLaunchKernelGGL((qkv_rope_cache_wide_kernel<HD, 2, 2>), g, dim3(256), 0, st, p);
+            else hipLaunchKernelGGL((qkv_rope_cache_wide_kernel<HD, 2, 4>), g, dim3(256), 0, st, p);
             return hipGetLastError();
         };
         switch (p.hd) {

@@ -192,3 +192,35 @@ def test_wide_accesses(n_seq, T, n_head, n_kv, hd, rot, neox, split, norm):
     print(f"[case] wide T{T} h{n_head}/{n_kv} hd{hd} rot{rot} neox{neox} split{split} norm{norm}", flush=True)
     _check(*_run_both(q, k, v, n_kv=n_kv, kv_len=L, rows=n_seq * L, table=table, rot=rot, neox=neox, table_split=split,
                       q_norm=w, k_norm=w), "wide accesses")
+
+
+@pytest.mark.parametrize("T,n_head,n_kv,hd,norm", [
+    (1025, 24, 8, 64, False),    # 5 waves a token: two tokens a workgroup, the last one alone
+    (395, 26, 13, 128, True),    # 13 waves
+    (733, 28, 14, 64, False),    # 7 waves: four tokens a workgroup, one in the last
+    (343, 30, 15, 128, True),    # 15 waves: ... three in the last
+])
+def test_tokens_per_workgroup(T, n_head, n_kv, hd, norm):
+    # the whole step against the same tokens in small steps, whose workgroups
+    # take one token each: the same arithmetic, so the same bits
+    first = 100
+    q, k, v = _case(1, T, n_head, n_kv, hd, seed=T)
+    table = torch.from_numpy(orc.rope_table(first + T, hd)).cuda()
+    w = torch.linspace(0.5, 1.5, hd, device="cuda") if norm else None
+    print(f"[case] tokens a workgroup T{T} h{n_head}/{n_kv} hd{hd} norm{norm}", flush=True)
+
+    def run(step):
+        qg = q.clone()
+        kc = torch.full((first + T, n_kv, hd), 7.0, dtype=torch.float16, device="cuda")
+        vc = kc.clone()
+        for t in range(0, T, step):
+            n = min(step, T - t)
+            qs = qg[:, t:t + n].contiguous()
+            attn.qkv_rope_cache(qs, k[:, t:t + n].contiguous(), v[:, t:t + n].contiguous(), kc, vc, n_kv=n_kv,
+                                kv_len=first + t + n, table=table, rot=hd, neox=True, q_norm=w, k_norm=w)
+            qg[:, t:t + n] = qs
+        torch.cuda.synchronize()
+        return qg, kc, vc
+
+    for a, b in zip(run(T), run(100)):
+        assert torch.equal(a, b)
