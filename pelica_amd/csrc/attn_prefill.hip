@@ -1347,67 +1347,16 @@ static int prefill_cus() {
     return n;
 }
 
-// How an 8-wave launch cuts its work: `split` 1 is one key group per
-// workgroup on all of its rows; each step halves a workgroup's rows and
-// doubles the number of workgroups: key groups 2, 4 and (head dim 64) 8, then
-// (16) eight groups with one row tile a wave; at head dim 128 the last (8) is
-// four groups of one wave, as LDS holds no more.  Few rows leave most CUs idle
-// otherwise: 512 gpt-oss tokens are 64 workgroups of 512 rows, and a full
-// layer at position 30K took 772 us with 1 group, 414 with 2, 278 with 4, 317
-// with 8 (512 workgroups: two generations); 256 Qwen3 tokens over 27K keys
-// (two rounds) 635 / 331 / 224 / 206; 64 gpt-oss tokens at 8K 204 / 110 / 62 / 40 /
-// 27.5.  Where the grid fills the chip anyway, groups only cost: each loads
-// its own keys (LDS writes beside the operand reads), and every workgroup
-// pays its start and its merge (4096 fresh gpt-oss tokens 147 / 164 / 205 /
-// 281 us).  So the split with the least estimated time is taken, from what
-// these shapes measured: us per key a group walks and us per workgroup, with
-// most CUs idle (lat) and with all of them busy (thr: lower clock, shared
-// memory rates).
-struct SplitCost {
-    float key_lat, wg_lat, key_thr, wg_thr;
-};
-constexpr SplitCost kSplitCost64[5] = {{.0244f, 3.5f, .0325f, 4.0f}, {.0246f, 5.5f, .0330f, 6.8f}, {.0285f, 6.0f, .0350f, 8.0f},
-                                       {.0300f, 6.0f, .0370f, 8.0f}, {.0250f, 3.0f, .0250f, 4.8f}};
-constexpr SplitCost kSplitCost128[4] = {{.0232f, 4.0f, .0375f, 4.0f}, {.0240f, 5.0f, .0385f, 7.0f}, {.0325f, 5.0f, .0407f, 8.0f},
-                                        {.0290f, 4.2f, .0270f, 5.0f}};
-
-static int prefill_split(const PrefillParams& p, int rows) {
-    const SplitCost* const cost = p.hd == 64 ? kSplitCost64 : kSplitCost128;
-    const int n_split = p.hd == 64 ? 5 : 4;
-    const double cus = prefill_cus();
-    // keys of the longest token block, and how many fewer the shortest walks
-    const double keys = p.state ? p.key_end - p.key_begin : p.kv_len;
-    const double spread = std::min<double>(p.state ? std::max(0, p.T - (p.kv_len - p.key_end)) : p.T, keys);
-    const long long same = (long long)p.n_kv * p.n_seq;  // blocks of one length
-    // (the last share's masked tail stays inside 32-bit offsets)
-    const bool fits = ((long long)p.kv_len + 512) * p.row_stride * 2 < 1LL << 32;
-    double best = 0;
-    int pick = 1;
-    for (int i = 0; i < n_split; ++i) {
-        const int split = 1 << i, TB = rows / split / p.hpk, kg = std::min(split, p.hd == 64 ? 8 : 4);
-        if (TB == 0 || (i > 0 && !fits)) break;
-        const long long n_tb = (p.T + TB - 1) / TB, n = n_tb * same;
-        auto walk = [&](long long b) { return (keys - (double)(b / same) / n_tb * spread) / kg; };  // block b, longest first
-        const SplitCost& c = cost[i];
-        // the longest block (at the clock of a chip whose CUs are busy that
-        // share of the time) ...
-        const double mean = (keys - spread / 2) / kg, busy = std::min(1.0, n / cus * mean / walk(0));
-        const double per_key = c.key_lat + (c.key_thr - c.key_lat) * std::max(0.0, 2 * busy - 1);
-        double t = walk(0) * per_key + c.wg_lat;
-        // ... all the work over all CUs ...
-        if (n >= cus) t = std::max(t, n / cus * (mean * c.key_thr + c.wg_thr));
-        // ... and g + 1 of the first g * cus + 1 blocks on one CU
-        for (int g = 1; g <= 8 && g * cus < n; ++g) t = std::max(t, (g + 1) * (walk((long long)(g * cus)) * c.key_lat + c.wg_lat));
-        if (i == 0 || 1.05 * t < best) best = t, pick = split;
-    }
-    return pick;
+static int split_of_call(const PrefillParams& p) {
+    return prefill_split({p.hd, p.hpk, p.n_kv, p.n_seq, p.T, p.kv_len, p.state ? p.key_begin : 0,
+                          p.state ? p.key_end : p.kv_len, p.window, p.f32, p.row_stride}, prefill_cus());
 }
 
 template <int HD, int RT, int NW, bool F32>
 static hipError_t launch_nw(const PrefillParams& p, hipStream_t st) {
     constexpr int ROWS = NW * RT * 32;
     if (p.hpk > ROWS) return hipErrorNotSupported;
-    const int split = NW == 8 && !p.ring_cap ? prefill_split(p, ROWS) : 1, KG = std::min(split, HD == 64 ? 8 : 4);
+    const int split = NW == 8 && !p.ring_cap ? split_of_call(p) : 1, KG = std::min(split, HD == 64 ? 8 : 4);
     const int TB = ROWS / split / p.hpk;
     const int n_tb = (p.T + TB - 1) / TB;
     const long long nblk = (long long)n_tb * p.n_kv * p.n_seq;

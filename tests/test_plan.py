@@ -1,27 +1,15 @@
-"""The kernels' address rules (pelica_amd/csrc/attn_plan.hpp), run on the host."""
-import ctypes
-import os
+"""The kernels' address rules and launch choices (pelica_amd/csrc/attn_plan.hpp),
+run on the host."""
 import random
-import subprocess
 
 import pytest
 
-HERE = os.path.dirname(os.path.abspath(__file__))
+from tests import plan_util
 
 
-@pytest.fixture(scope="session")
-def plan(tmp_path_factory):
-    so = str(tmp_path_factory.mktemp("plan") / "plan.so")
-    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-o", so,
-                    os.path.join(HERE, "plan_shim.cpp")], check=True)
-    lib = ctypes.CDLL(so)
-    u32, i32 = ctypes.c_uint32, ctypes.c_int32
-    lib.tile_base.restype = u32
-    lib.tile_base.argtypes = [i32, i32, u32]
-    lib.range_shift.argtypes = [i32, i32]
-    lib.burst_offset.restype = u32
-    lib.burst_offset.argtypes = [u32, u32, u32, i32, i32]
-    return lib
+@pytest.fixture
+def plan():
+    return plan_util.load()
 
 
 def _spans():
@@ -80,3 +68,59 @@ def test_key_range_blocks_start_at_its_rows(plan):
         assert row >= 0
         off = plan.burst_offset(lane_off, b, per_load * stride, j, e)
         assert off + 1024 * e == row * stride + lane % (hd // 8) * 16
+
+
+# us of every split (1, 2, 4, ...), as measured on an MI355X
+_MEASURED = [
+    # windows of several thousand keys: a block walks its window, not the cache
+    (dict(hd=128, n_head=40, n_kv=8, T=1024, kv_len=20688, window=1100), (37.1, 50.4, 49.4, 74.9)),
+    (dict(hd=128, n_head=40, n_kv=8, T=1024, kv_len=18369, window=8000, f32=True), (197.9, 235.4, 225.0, 335.2)),
+    (dict(hd=64, n_head=24, n_kv=8, T=1024, kv_len=24149, window=1500), (54.5, 34.2, 24.9, 41.4, 39.1)),
+    # one chunk of keys: nothing to divide
+    (dict(hd=64, n_head=64, n_kv=8, T=4, kv_len=21, f32=True), (7.2, 9.0, 10.2, 10.9, 8.7)),
+    (dict(hd=64, n_head=24, n_kv=8, T=16, kv_len=16, f32=True), (7.5, 9.4, 10.7, 11.7, 8.5)),
+    # ... but the queries to bring in
+    (dict(hd=128, n_head=32, n_kv=2, T=16, kv_len=16, f32=True), (12.7, 12.3, 11.9, 9.3)),
+    # kv heads that are no multiple of the XCDs: some get the long blocks
+    (dict(hd=128, n_head=32, n_kv=2, T=558, kv_len=558, n_seq=2, f32=True), (26.7, 32.6, 40.1, 46.7)),
+    (dict(hd=128, n_head=32, n_kv=4, T=1176, kv_len=1176), (36.6, 39.9, 39.7, 62.3)),
+    # few rows over many keys
+    (dict(hd=64, n_head=64, n_kv=8, T=512, kv_len=30512, f32=True), (772., 414., 278., 317., 400.)),
+    (dict(hd=128, n_head=32, n_kv=4, T=256, kv_len=27000, keys=(0, 16384)), (385., 200., 136., 125.)),
+    (dict(hd=64, n_head=64, n_kv=8, T=64, kv_len=8192), (204., 110., 62., 40., 27.5)),
+    # a full chip
+    (dict(hd=64, n_head=64, n_kv=8, T=4096, kv_len=4096), (147., 164., 205., 281., 400.)),
+]
+
+
+@pytest.mark.parametrize("call,times", _MEASURED)
+def test_split_is_a_fast_one(call, times):
+    split = plan_util.prefill_split(**call)
+    assert times[split.bit_length() - 1] <= 1.1 * min(times), split
+
+
+def test_split_counts_the_keys_a_window_shows():
+    # keys before every window change nothing
+    rng = random.Random(4)
+    for _ in range(500):
+        n_head, n_kv, hd = rng.choice([(64, 8, 64), (32, 4, 128), (40, 8, 128), (16, 16, 128), (24, 8, 64)])
+        T, window, f32 = rng.randint(1, 3000), rng.randint(1025, 9000), rng.random() < 0.5
+        near = plan_util.prefill_split(hd, n_head, n_kv, T, T + window, window=window, f32=f32)
+        far = plan_util.prefill_split(hd, n_head, n_kv, T, T + window + rng.randint(1, 200000), window=window, f32=f32)
+        assert near == far, (n_head, n_kv, hd, T, window)
+
+
+def test_split_is_one_the_launch_has():
+    rng = random.Random(5)
+    for _ in range(3000):
+        hd = rng.choice((64, 128))
+        rows = 512 if hd == 64 else 256
+        hpk = rng.choice((1, 2, 3, 5, 8, 16, 40, 100, rows))
+        n_kv, n_seq, T = rng.randint(1, 40), rng.choice((1, 1, 2, 9, 64)), int(2 ** rng.uniform(0, 17))
+        kv_len = T + rng.choice((0, rng.randint(0, 300000)))
+        b = rng.randint(1, kv_len)
+        keys = rng.choice((None, (rng.randrange(b), b)))
+        split = plan_util.prefill_split(hd, hpk * n_kv, n_kv, T, kv_len, n_seq=n_seq, keys=keys,
+                                        window=rng.choice((0, 0, 1025, 5000)), f32=rng.random() < 0.5,
+                                        cus=rng.choice((256, 304, 38, 1)))
+        assert split in ((1, 2, 4, 8, 16) if hd == 64 else (1, 2, 4, 8)) and rows // split >= hpk
