@@ -326,7 +326,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kDecode
     // key range's rows start at position kr_lo, the first of a split: no
     // block starts below it.)
     const uint32_t stride_b = (uint32_t)p.row_stride * 2;
-    const uint32_t nrec = (RING ? (uint32_t)p.ring_cap : (uint32_t)(min(len, p.kr_hi) - p.kr_lo)) * stride_b;
+    // (a ring that has not wrapped: the rows after len were never written)
+    const uint32_t nrec = (uint32_t)(RING ? min(len, p.ring_cap) : min(len, p.kr_hi) - p.kr_lo) * stride_b;
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(p.k + row0 * p.row_stride + (size_t)kvh * HD), (short)0, (int)nrec, kBufferFlags);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(

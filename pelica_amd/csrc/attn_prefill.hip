@@ -119,8 +119,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     // streaming: K0 K1 V0 V1; resident: K[NRES] V[NRES] and a zero tile
     constexpr int NBUF = NRES ? 2 * NRES + 1 : 4;
     static_assert(!NRES || (!ROUND && KG == 1 && TK == 64), "resident tiles: whole-cache launches, one key group");
-    // (a share's chunks past klast: zeros past a linear cache's rows, but a
-    // ring's rows there may never have been written)
+    // (a share's chunks past klast: zeros past a linear cache's rows, but old
+    // keys in a ring)
     static_assert(!RING || KG == 1, "key groups: linear caches");
     // after the tile loop the f16 output of each wave is staged here
     constexpr int OUT_WAVE = RT * 32 * HD * 2;  // bytes of one wave's output rows
@@ -164,8 +164,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     const int klast = min(pos_last, kend - 1);  // the last key a row sees
     // every row sees every key from lo_all to hi_all of this launch
     const int lo_all = ROUND ? max(lo_last, kbeg) : lo_last, hi_all = ROUND ? min(pos_first, kend - 1) : pos_first;
-    // (key groups: rows past klast, in a share's tail, read as zeros too)
-    const uint32_t nrec = (RING ? (uint32_t)p.ring_cap : (uint32_t)max(0, (KG > 1 ? klast + 1 : kend) - kbeg)) * stride_b;
+    // (key groups: rows past klast, in a share's tail, read as zeros too; a
+    // ring that has not wrapped: the rows after len were never written)
+    const uint32_t nrec = (uint32_t)(RING ? min(len, p.ring_cap) : max(0, (KG > 1 ? klast + 1 : kend) - kbeg)) * stride_b;
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(p.k + row0 * p.row_stride + (size_t)kvh * HD), (short)0, (int)nrec, kBufferFlags);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
@@ -937,7 +938,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int qoff0 = len - p.T;  // position of token 0
     const uint32_t stride_b = (uint32_t)p.row_stride * 2;
     // (ring caches: key j sits in row j % ring_cap)
-    const uint32_t nrec = (uint32_t)(RING ? p.ring_cap : len) * stride_b;
+    // (a ring that has not wrapped: the rows after len were never written)
+    const uint32_t nrec = (uint32_t)(RING ? min(len, p.ring_cap) : len) * stride_b;
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(p.k + row0 * p.row_stride + (size_t)kvh * HD), (short)0, (int)nrec, kBufferFlags);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
