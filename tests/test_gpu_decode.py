@@ -382,3 +382,17 @@ def test_given_workspace_is_used_replaced_or_refused_as_before():
         with pytest.raises(attn.AttnError) as e:
             attn.decode(inp.q, inp.k, inp.v, workspace=ws, **{**kw, **bad})
         assert e.value.code == attn.EINVAL
+
+
+def test_default_stream_argument_is_the_current_stream():
+    q = torch.zeros(1, 1, 64, 64, device="cuda")
+    kv = torch.zeros(64, 8, 64, dtype=torch.float16, device="cuda")
+    attn.decode(q, kv, kv, n_kv=8, kv_len=64)  # (from here on the handle comes without a Stream object)
+    default = torch.cuda.default_stream().cuda_stream or None
+    assert attn._stream_ptr(None) == default
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert attn._stream_ptr(None) == side.cuda_stream != default
+        assert attn._stream_ptr(torch.cuda.default_stream()) == default
+    assert attn._stream_ptr(None) == default
+    torch.cuda.synchronize()

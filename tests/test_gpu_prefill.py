@@ -252,3 +252,49 @@ def test_short_window_row_tiles(T, L, window, n_seq, n_head, f32):
     if f32:
         inp.q = inp.q.float()
     assert_close(as_f64(gpu_run(inp)), ref, what="short window")
+
+
+# every form of the 8-wave prompt kernel: splits 1, 2, 4, 8 and (head dim 64)
+# 16, whole and in rounds, for both query types.  The choice is asserted, so
+# that costs fitted anew cannot move a case to another form unnoticed.
+@pytest.mark.parametrize("hd,n_head,n_kv,T,L,bounds,splits", [
+    (64, 64, 8, 2300, 2300, None, [1]),
+    (64, 64, 8, 700, 720, None, [2]),
+    (64, 64, 8, 300, 311, None, [4]),
+    (64, 64, 8, 250, 1250, None, [8]),
+    (64, 64, 8, 20, 1500, None, [16]),
+    (128, 32, 4, 2100, 2100, None, [1]),
+    (128, 32, 4, 1000, 1000, None, [2]),
+    (128, 32, 4, 500, 520, None, [4]),
+    (128, 32, 4, 256, 256, None, [8]),
+    (64, 64, 8, 2100, 2500, [0, 900, 2500], [1, 2]),
+    (64, 64, 8, 900, 2200, [0, 1100, 2200], [2, 2]),
+    (64, 64, 8, 512, 2000, [0, 1000, 2000], [4, 4]),
+    (64, 64, 8, 250, 4500, [0, 1500, 3000, 4500], [8, 8, 8]),
+    (64, 64, 8, 40, 3000, [0, 1, 700, 2980, 3000], [16, 16, 16, 16]),
+    (128, 32, 4, 2100, 2500, [0, 1300, 2500], [1, 1]),
+    (128, 32, 4, 1000, 2500, [0, 1300, 2500], [2, 2]),
+    (128, 32, 4, 490, 2000, [0, 1000, 1510, 2000], [4, 4, 4]),
+    (128, 32, 4, 100, 5000, [0, 777, 3000, 5000], [8, 8, 8]),
+])
+@pytest.mark.parametrize("f32", [False, True])
+def test_every_split(hd, n_head, n_kv, T, L, bounds, splits, f32):
+    from tests import plan_util
+    from tests.test_gpu_prefill_rounds import run_rounds
+
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    keys = list(zip(bounds, bounds[1:])) if bounds else [None]
+    assert [plan_util.prefill_split(hd, n_head, n_kv, T, L, keys=k, f32=f32, cus=cus) for k in keys] == splits
+    cfg = wl.AttnConfig("psp", "prefill", n_head, n_kv, hd, L, q_tokens=T, sinks=True, seed=hd + T + L)
+    inp = wl.make_inputs(cfg, "cuda")
+    print(f"[case] splits {splits} hd{hd} T{T} L{L} {bounds} f32 {f32}", flush=True)
+    ref = as_f64(oracle_run(inp))
+    if f32:
+        inp.q = inp.q.float()
+    if bounds:
+        out, state = run_rounds(inp, bounds)
+        assert torch.isfinite(state).all()
+    else:
+        out = gpu_run(inp)
+    assert out.dtype == inp.q.dtype
+    assert_close(as_f64(out), ref, what="every split")

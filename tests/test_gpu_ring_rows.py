@@ -44,3 +44,20 @@ def test_rows_never_written(kind, hd, n_head, n_kv, T, L, window, cap, f32):
         inp.q = inp.q.float()
     got = gpu_run(inp, ring_cap=cap, k=_ring(inp, L, cap, inp.k), v=_ring(inp, L, cap, inp.v))
     assert_close(as_f64(got), ref, what="ring rows")
+
+
+@pytest.mark.parametrize("T,L,window,cap,f32", [
+    (100, 2000, 500, 607, False),   # one row tile a wave over streamed tiles, a ring that has wrapped
+    (300, 1500, 1000, 1300, True),
+    (40, 900, 200, 256, False),     # tiles that wrap inside
+    (1, 400, 700, 701, True),
+])
+def test_streamed_ring_tiles_of_one_row_tile(T, L, window, cap, f32):
+    cfg = wl.AttnConfig("ringst", "prefill", 64, 8, 64, L, q_tokens=T, window=window, sinks=True, seed=T + cap)
+    inp = wl.make_inputs(cfg, "cuda")
+    print(f"[case] streamed ring tiles T{T} L{L} window{window} cap{cap} f32 {f32}", flush=True)
+    ref = as_f64(oracle_run(inp))
+    if f32:
+        inp.q = inp.q.float()
+    got = gpu_run(inp, ring_cap=cap, k=_ring(inp, L, cap, inp.k), v=_ring(inp, L, cap, inp.v))
+    assert_close(as_f64(got), ref, what="streamed ring tiles")
