@@ -131,7 +131,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(kPrefil
     __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES];
 
     // XCD-aware block order: dispatch goes round-robin over the 8 XCDs, so
-    // give each XCD a contiguous range of logical blocks (same kv head)
+    // give each XCD a contiguous range of logical blocks (8 kv heads: one
+    // each; with 4, the long or the short half of a head's blocks, which
+    // prefill_split counts)
     const int nblk = gridDim.x;
     int bid = blockIdx.x;
     if ((nblk & 7) == 0) bid = (bid & 7) * (nblk >> 3) + (bid >> 3);

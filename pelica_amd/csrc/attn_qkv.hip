@@ -6,8 +6,11 @@
 //
 // Head slots [0, n_head) are q heads, then n_kv k heads, then n_kv v heads;
 // a lane holds 4 consecutive elements of its slot (16-byte accesses), a wave
-// 64/(hd/4) slots of a few consecutive tokens.  The norm is a reduction over the slot's lanes; the
-// rotation reads each element's partner through the slot's LDS row.
+// 64/(hd/4) slots.  The norm is a reduction over the slot's lanes.  Two
+// kernels: where every access can be 16 bytes wide (launch_qkv's rule) a wave
+// takes one token and one or two such groups of slots, and a rotation partner
+// comes from its lane's registers; else a few consecutive tokens, with the
+// partners through the slot's LDS row.
 // HBM-bound: every byte is touched once.
 #include <type_traits>
 
@@ -162,7 +165,7 @@ __global__ __launch_bounds__(256) void qkv_rope_cache_kernel(QkvParams p) {
     }
 }
 
-// The same step where every access can be 16 bytes wide (QkvParams::wide): a
+// The same step where every access can be 16 bytes wide (launch_qkv): a
 // wave takes one token and IT groups of 64/(HD/4) consecutive heads; the
 // token's rotation is loaded in 16-byte pieces, once for all of its groups,
 // and a rotation partner comes from its lane's registers, not through LDS.
@@ -249,7 +252,6 @@ __global__ __launch_bounds__(256) void qkv_rope_cache_wide_kernel(QkvParams p) {
                 for (int i = 0; i < 4; ++i) {
                     const bool second = p.neox ? hi : (i & 1) != 0;
                     r[i] = second ? z[i] * sn[i] + y[i] * c[i] : y[i] * c[i] - z[i] * sn[i];
-                    if (!p.neox && e0 + i >= p.rot) r[i] = y[i];
                 }
                 y = r;
             }
