@@ -85,11 +85,12 @@ _MEASURED = [
     (dict(hd=128, n_head=32, n_kv=2, T=558, kv_len=558, n_seq=2, f32=True), (26.7, 32.6, 40.1, 46.7)),
     (dict(hd=128, n_head=32, n_kv=4, T=1176, kv_len=1176), (36.6, 39.9, 39.7, 62.3)),
     # few rows over many keys
-    (dict(hd=64, n_head=64, n_kv=8, T=512, kv_len=30512, f32=True), (772., 414., 278., 317., 400.)),
-    (dict(hd=128, n_head=32, n_kv=4, T=256, kv_len=27000, keys=(0, 16384)), (385., 200., 136., 125.)),
-    (dict(hd=64, n_head=64, n_kv=8, T=64, kv_len=8192), (204., 110., 62., 40., 27.5)),
+    (dict(hd=64, n_head=64, n_kv=8, T=512, kv_len=19817, f32=True), (496.7, 269.4, 190.9, 219.7, 276.9)),
+    (dict(hd=128, n_head=32, n_kv=4, T=85, kv_len=10815, keys=(825, 10815), f32=True), (230.1, 124.3, 94.2, 75.5)),
+    (dict(hd=128, n_head=32, n_kv=4, T=518, kv_len=6246, keys=(3439, 6246)), (77.8, 48.3, 59.0, 69.6)),
+    (dict(hd=64, n_head=64, n_kv=8, T=25, kv_len=4270), (110.6, 61.9, 39.9, 26.1, 18.5)),
     # a full chip
-    (dict(hd=64, n_head=64, n_kv=8, T=4096, kv_len=4096), (147., 164., 205., 281., 400.)),
+    (dict(hd=64, n_head=64, n_kv=8, T=3196, kv_len=3196), (107.2, 121.3, 155.7, 218.3, 273.1)),
 ]
 
 
